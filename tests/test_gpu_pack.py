@@ -98,3 +98,47 @@ def test_malformed_buffers_are_errors(codec):
         codec.embeddings_from_packed(bytes(b), 128)
     except RuntimeError:
         pass
+
+
+def _or_refused(fn, *args):
+    try:
+        return fn(*args)
+    except (RuntimeError, ValueError):
+        return "refused"
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (21, 3), (64, 1), (13, 5), (127, 1), (127, 8), (341, 3), (512, 2),
+                                       (205, 5), (344, 3), (1024, 2), (73, 57)])
+@pytest.mark.parametrize("kind", ["smooth", "two", "flat"])
+def test_coder_lengths_and_histograms(codec, rows, cols, kind):
+    """Value counts around the coder's steps (8 and 64 symbols, 1024 staged positions) on histograms
+    from one dominant symbol to hundreds of rare ones; what the oracle refuses is refused."""
+    rng = np.random.default_rng(rows)
+    if kind == "two":  # a constant with one step: few nonzero coefficients
+        x = np.full((rows, cols), 0.5, np.float32)
+        x[rows // 2:] = 0.51
+    elif kind == "flat":
+        x = rng.uniform(-0.4, 0.4, (rows, cols)).astype(np.float32)
+    else:
+        x = _emb(rows, cols, rows) * rng.uniform(0.1, 0.9, (rows, 1)).astype(np.float32)
+    buf = _or_refused(orc.embeddings_to_packed, x)
+    assert _or_refused(codec.embeddings_to_packed, x) == buf
+    if buf != "refused":
+        got, want = codec.embeddings_from_packed(buf, cols), orc.embeddings_from_packed(buf, cols)
+        assert got.view(np.uint32).tolist() == want.view(np.uint32).tolist()
+
+
+@pytest.mark.parametrize("delta", [-1, -3, 1])
+def test_histogram_totals_other_than_the_slots(codec, delta):
+    """A frequency changed in the stored histogram: slots left uncovered decode as the oracle
+    decodes them (or both refuse); a total above 4096 is refused."""
+    b = bytearray(orc.embeddings_to_packed(_emb(40, 128, 9)))
+    at = 4 + 128 + 2 + 2  # first symbol's frequency
+    f = int.from_bytes(b[at:at + 2], "little") + delta
+    b[at:at + 2] = f.to_bytes(2, "little")
+    got, want = (_or_refused(fn, bytes(b), 128) for fn in (codec.embeddings_from_packed, orc.embeddings_from_packed))
+    if isinstance(want, str):
+        assert isinstance(got, str)
+    else:
+        assert got.view(np.uint32).tolist() == want.view(np.uint32).tolist()
+    assert delta < 0 or isinstance(got, str)

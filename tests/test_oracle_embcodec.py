@@ -282,3 +282,31 @@ def test_packed_decoder_rejects_malformed():
         orc.embeddings_from_packed(buf + b"\0", 128)  # leftover bytes
     with pytest.raises(ValueError):
         orc.embeddings_from_packed(buf[:-3], 128)  # truncated stream
+
+
+@pytest.mark.parametrize("freqs", [range(1, 70), range(70, 4097, 13), range(4060, 4097)])
+def test_rans_step_in_f64_is_exact(freqs):
+    """The encoder's state step as k_pack.hip takes it (x = A 2^32 + B, divisions by a reciprocal
+    rounded up) equals the integer step for every state a renormalised coder can hold: random
+    ones, the ends of the range and the neighbours of multiples of the frequency."""
+    rng = np.random.default_rng(5)
+    for f in freqs:
+        hi = f << 51
+        base = [int(v) for v in rng.integers(1 << 31, hi, 40, dtype=np.uint64)]
+        xs = sorted({min(max(v + d, 1 << 31), hi - 1) for v in base + [1 << 31, hi - 1, 1 << 32, hi >> 1]
+                     for v in (v, v // f * f) for d in (-1, 0, 1)})
+        start = min(4096 - f, int(rng.integers(0, 4097 - f)))
+        rf = 1.0 / f
+        if rf.as_integer_ratio()[0] * f < rf.as_integer_ratio()[1]:  # below 1 / f: the next one up
+            rf = float(np.nextafter(rf, 2.0))
+        A = np.array([v >> 32 for v in xs], np.float64)
+        B = np.array([v & 0xffffffff for v in xs], np.float64)
+        assert not (A * rf >= 2.0 ** 19).any()  # the renormalisation test: x < freq 2^51
+        assert ((float(f * (1 << 19)) * rf) >= 2.0 ** 19)
+        qa = np.floor(A * rf)
+        t = (A - qa * f) * 2.0 ** 32 + B
+        qb = np.floor(t * rf)
+        u = t + start + qb * (4096 - f)
+        c = np.floor(u * 2.0 ** -32)
+        got = [(int(a) << 32) + int(b) for a, b in zip(qa * 4096 + c, u - c * 2.0 ** 32)]
+        assert got == [(v // f << 12) + v % f + start for v in xs]

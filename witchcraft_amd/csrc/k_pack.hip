@@ -10,10 +10,11 @@
 //           -> pk_haar_cols (column transform in LDS, 8 columns per workgroup)
 //           -> pk_quant (max |x| < 1, symbols round(29 x) folded to unsigned, histogram over
 //              the used symbol range in 8192-bin LDS passes, scale_histogram)
-//           -> pk_rans_enc (one workgroup per window: per-position coder parameters staged in
-//              LDS in parallel, then the wave-uniform state loop writes 32-bit words backwards)
+//           -> pk_rans_enc (one workgroup per window: one wave runs the state loop, the state as
+//              two f64 integers, and writes 32-bit words backwards; the others stage its
+//              per-position parameters in LDS)
 //           -> pk_assemble (header pieces and stream copied to host-computed offsets).
-//   decode: pk_rans_dec (decode table in LDS, wave-uniform state loop, values in reverse)
+//   decode: pk_rans_dec (slot table in LDS, one wave runs the state loop, values in reverse)
 //           -> pk_haar_rows<inverse> -> pk_haar_cols<inverse> -> pk_unpermute_norm.
 // rANS64 has one state per window and the format fixes one stream per window, so the coder
 // runs one stream per workgroup; windows run in parallel.
@@ -339,82 +340,79 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
   }
 }
 
-// rANS64 encoder symbol (rans64.rs:41-87): reciprocal of freq with ceil(log2 freq) shift.
-struct EncSym {
-  unsigned long long rcp;
-  uint32_t bias, freq_shift;  // freq | (rcp_shift << 16)
+// ---- encode 5: rANS64, one workgroup per window.  The state x is a serial chain over the
+// window's symbols, so what bounds the launch is the latency of one step of one wave, not a
+// unit: 65,536 steps for 512 rows of 128.  The step, with f = freq and g = 4096 - f, is
+//   q = floor(x / f),  x' = x + start + q g
+// (the reference multiplies by a 64-bit reciprocal, rans64.rs:41-87; both divide exactly).  In
+// integers the 64 x 64-bit high product alone is seven multiplies and their carries on the
+// scalar unit.  f64 is full rate here, so x lives as two f64 integers, x = A 2^32 + B (A < 2^31,
+// B < 2^32), and a step is 12 f64 instructions, each exact:
+//   qA = floor(A / f), rA = A - qA f, t = rA 2^32 + B < 2^44, qB = floor(t / f) < 2^32,
+//   u = t + start + qB g < 2^44, c = floor(u / 2^32), B' = u - c 2^32, A' = 4096 qA + c.
+// floor(v / f) = floor(v * rf) with rf = 1 / f rounded up: a multiple of f cannot fall below its
+// quotient, and any other v / f lies at least 1 / f >= 2^-12 under the next integer, against an
+// error of at most 2^32 * 2^-51.  The renormalisation test x >= f 2^51 is A / f >= 2^19, i.e.
+// A * rf >= 2^19 by the same argument.  Wave 0 runs the chain (all lanes alike); the other
+// waves gather the next chunk's per-position parameters into LDS meanwhile.
+// 48 windows of up to 512 rows: 8.07 -> 3.25 ms. ----
+constexpr int ENC_CHUNK = 1024;
+struct EncPos {
+  double rf, f, g, start;
 };
 
-__device__ __forceinline__ EncSym enc_sym(uint32_t cum, uint32_t freq) {
-  EncSym e;
-  if (freq < 2) {
-    e.rcp = ~0ull;
-    e.bias = cum + (RANS_TOTAL - 1);
-    e.freq_shift = freq;
-  } else {
-    uint32_t shift = 0;
-    while (freq > (1u << shift)) shift++;
-    // ceil(2^(shift + 63) / freq) in 128-bit arithmetic: 2^(shift+63) = hi * 2^64 with hi = 2^(shift-1)
-    const unsigned long long hi = 1ull << (shift - 1);
-    const unsigned long long q_hi = hi / freq, r_hi = hi % freq;  // (r_hi * 2^64) / freq next
-    // long division of r_hi * 2^64 by freq (freq < 2^13): 4 steps of 16 bits
-    unsigned long long q_lo = 0, r = r_hi;
-    for (int k = 0; k < 4; k++) {
-      r = (r << 16);
-      q_lo = (q_lo << 16) | (r / freq);
-      r = r % freq;
-    }
-    (void)q_hi;  // 2^(shift+63) / freq < 2^64 since freq > 2^(shift-1): q_hi == 0
-    e.rcp = q_lo + (r != 0 ? 1ull : 0ull);
-    e.bias = cum;
-    e.freq_shift = freq | ((shift - 1) << 16);
+// Exclusive prefix sums of the window's m frequencies (freq(i), i < m <= 4096) by 256 threads, 16
+// consecutive entries each, written as start | freq << 16; returns the total.
+template <class Freq>
+__device__ __forceinline__ uint32_t pk_starts(int m, Freq freq, uint32_t* out, uint32_t* red) {
+  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
+  uint32_t f[16], sum = 0;
+#pragma unroll
+  for (int j = 0; j < 16; j++) {
+    f[j] = 16 * tid + j < m ? freq(16 * tid + j) : 0;
+    sum += f[j];
   }
-  return e;
+  uint32_t incl = sum;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  if (lane == 63) red[wid] = incl;
+  __syncthreads();
+  uint32_t at = incl - sum, total = 0;
+  for (int i = 0; i < 4; i++) {
+    if (i < wid) at += red[i];
+    total += red[i];
+  }
+#pragma unroll
+  for (int j = 0; j < 16; j++) {
+    if (16 * tid + j < m) out[16 * tid + j] = (at & 0xffffu) | (f[j] << 16);
+    at += f[j];
+  }
+  __syncthreads();
+  return total;
 }
 
-// ---- encode 5: rANS64, one workgroup per window.  Encoder parameters of the window's m
-// symbols go to LDS; chunks of per-position parameters are staged in LDS by all threads; wave 0
-// runs the (wave-uniform) state loop and writes each 32-bit word with lane 0. ----
-constexpr int ENC_CHUNK = 2048;
 __global__ __launch_bounds__(256) void pk_rans_enc(const uint16_t* __restrict__ syms, PkWin* __restrict__ win,
                                                     int cols, const uint32_t* __restrict__ pairs_scratch,
                                                     uint8_t* __restrict__ data_scratch) {
-  __shared__ EncSym table[4096];
+  __shared__ uint32_t table[RANS_TOTAL];  // start | freq << 16
   __shared__ uint16_t sym2idx[HBINS];
-  __shared__ EncSym stage[ENC_CHUNK];
-  __shared__ int fail;
+  __shared__ __attribute__((aligned(16))) EncPos stage[2][ENC_CHUNK + 8];
+  __shared__ uint32_t red[4];
   PkWin& w = win[blockIdx.x];
   if (w.err) return;  // uniform
   const int m = w.m, n = w.rows * cols, tid = threadIdx.x;
   const uint32_t* pairs = pairs_scratch + (size_t)blockIdx.x * 4096 * 2;
-  if (tid == 0) {
-    uint32_t cum = 0;
-    for (int i = 0; i < m; i++) {
-      table[i].bias = cum;  // cumulative start, turned into EncSym below
-      cum += pairs[2 * i + 1];
-    }
-    fail = 0;
-  }
+  const uint16_t* sy = syms + (size_t)w.row0 * cols;
+  pk_starts(m, [&](int i) { return pairs[2 * i + 1]; }, table, red);
+  for (int i = tid; i < m; i += 256)
+    if (pairs[2 * i] < HBINS) sym2idx[pairs[2 * i]] = (uint16_t)i;
   __syncthreads();
-  for (int i = tid; i < m; i += 256) {
-    const uint32_t sym = pairs[2 * i], cum = table[i].bias;
-    table[i] = enc_sym(cum, pairs[2 * i + 1]);
-    if (sym < HBINS) sym2idx[sym] = (uint16_t)i;
-  }
-  __syncthreads();
-  // The encoder pushes symbols 0..n-1 in order.  The reference writes them backwards into a
-  // buffer of 2n bytes (renormalisation needs 4 free bytes, the final flush 8, else it
-  // panics); here word j (the j-th emitted) goes to out_words[cap_w - 1 - j] and the state
-  // just before the last word, so the stream is contiguous: state, words k-1 .. 0.
-  uint32_t* out_words = reinterpret_cast<uint32_t*>(data_scratch + w.data);
-  const long long cap_w = n / 2 + 4;
-  long long k = 0;               // words emitted
-  const long long cap_b = 2LL * n;  // the reference's buffer size in bytes
-  unsigned long long x = RANS_L;
-  for (int c0 = 0; c0 < n; c0 += ENC_CHUNK) {
-    const int cn = min(ENC_CHUNK, n - c0);
-    for (int i = tid; i < cn; i += 256) {
-      const uint32_t s = syms[(size_t)w.row0 * cols + c0 + i];
+  auto fill = [&](int c0, int t0, int nt) {  // positions [c0, c0 + ENC_CHUNK) by threads t0 .. t0 + nt
+    EncPos* st = stage[(c0 / ENC_CHUNK) & 1];
+    for (int i = t0; i < min(ENC_CHUNK, n - c0); i += nt) {
+      const uint32_t s = sy[c0 + i];
       int kk;
       if (s < HBINS) {
         kk = sym2idx[s];
@@ -427,59 +425,82 @@ __global__ __launch_bounds__(256) void pk_rans_enc(const uint16_t* __restrict__ 
         }
         kk = lo;
       }
-      stage[i] = table[kk];
+      const uint32_t sf = table[kk];
+      const double f = (double)(sf >> 16);
+      double r = 1.0 / f;
+      if (__builtin_fma(r, f, -1.0) < 0.0) r = __longlong_as_double(__double_as_longlong(r) + 1);
+      st[i] = EncPos{r, f, 4096.0 - f, (double)(sf & 0xffffu)};
     }
-    __syncthreads();
-    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0 && !fail) {
-      // Wave 0 runs the coder; every value below is wave-uniform (parameters pass through
-      // readfirstlane), so the state lives in scalar registers and the loop branches on the
-      // scalar unit.  Parameters of the next 4 positions are read from LDS one group ahead.
-      EncSym nx[4];
+  };
+  fill(0, tid, 256);
+  __syncthreads();
+  // The encoder pushes symbols 0..n-1 in order.  The reference writes them backwards into a
+  // buffer of 2n bytes (renormalisation needs 4 free bytes, the final flush 8, else it
+  // panics); here word j (the j-th emitted) goes to out_words[cap_w - 1 - j] and the state
+  // just before the last word, so the stream is contiguous: state, words k-1 .. 0.
+  uint32_t* out_words = reinterpret_cast<uint32_t*>(data_scratch + w.data);
+  const int cap_w = n / 2 + 4, cap_k = (2 * n) / 4;  // the reference's buffer holds cap_k whole words
+  int k = 0;                                         // words emitted; past cap_k: the window fails
+  double A = 0.0, B = (double)RANS_L;
+  // One step of (a, b) given z = a * rf.
+  auto push = [](const EncPos& e, double a, double b, double z, double& an, double& bn) {
+    const double qa = __builtin_floor(z);
+    const double ra = __builtin_fma(-qa, e.f, a);
+    const double bs = b + e.start;
+    const double t = __builtin_fma(ra, 4294967296.0, b), ts = __builtin_fma(ra, 4294967296.0, bs);
+    const double qb = __builtin_floor(t * e.rf);
+    const double u = __builtin_fma(qb, e.g, ts);
+    const double c = __builtin_floor(u * 0x1p-32);
+    bn = __builtin_fma(c, -4294967296.0, u);
+    an = __builtin_fma(qa, 4096.0, c);
+  };
+  // The step is taken before the renormalisation test is known (a vector compare takes ~16 clk to
+  // reach the scalar branch) and taken again in the 5% of positions that emit a word.
+  auto step = [&](const EncPos& e) {
+    double an, bn;
+    const double z = A * e.rf;
+    const unsigned long long full = __builtin_amdgcn_ballot_w64(z >= 524288.0);  // all lanes alike
+    push(e, A, B, z, an, bn);
+    asm volatile("" : "+v"(an), "+v"(bn));  // taken here, not behind the branch
+    if (__builtin_expect(full != 0, 0)) {
+      out_words[cap_w - 1 - min(k, cap_k)] = (uint32_t)B;  // a full buffer fails the window below
+      k++;
+      push(e, 0.0, A, 0.0, an, bn);
+    }
+    A = an;
+    B = bn;
+  };
+  for (int c0 = 0; c0 < n; c0 += ENC_CHUNK) {
+    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
+      const EncPos* st = stage[(c0 / ENC_CHUNK) & 1];
+      const int cn = min(ENC_CHUNK, n - c0), full = cn & ~7;
+      EncPos nx[8];  // the next 8 positions, read from LDS while 8 are coded
 #pragma unroll
-      for (int j = 0; j < 4; j++) nx[j] = stage[min(j, cn - 1)];
-      bool ok = true;
-      for (int i = 0; i < cn && ok; i += 4) {
-        EncSym cu[4];
+      for (int j = 0; j < 8; j++) nx[j] = st[j];
+      for (int i = 0; i < full && k <= cap_k; i += 8) {
+        EncPos cu[8];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < 8; j++) {
           cu[j] = nx[j];
-          nx[j] = stage[min(i + 4 + j, cn - 1)];
+          nx[j] = st[i + 8 + j];  // up to 8 past the chunk: inside the array, not used
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (i + j >= cn || !ok) break;
-          const uint32_t fs = __builtin_amdgcn_readfirstlane(cu[j].freq_shift);
-          const uint32_t bias = __builtin_amdgcn_readfirstlane(cu[j].bias);
-          const uint32_t rlo = __builtin_amdgcn_readfirstlane((uint32_t)cu[j].rcp);
-          const uint32_t rhi = __builtin_amdgcn_readfirstlane((uint32_t)(cu[j].rcp >> 32));
-          const uint32_t freq = fs & 0xffffu, shift = fs >> 16;
-          const unsigned long long rcp = ((unsigned long long)rhi << 32) | rlo;
-          const unsigned long long x_max = (1ull << 51) * freq;  // ((L >> 12) << 32) * freq
-          while (x >= x_max) {
-            if (cap_b - 4 * k < 4) {
-              ok = false;
-              break;
-            }
-            if (tid == 0) out_words[cap_w - 1 - k] = (uint32_t)x;
-            k++;
-            x >>= 32;
-          }
-          const unsigned long long q = __umul64hi(x, rcp) >> shift;
-          x = x + bias + q * (unsigned long long)(RANS_TOTAL - freq);
-        }
+        for (int j = 0; j < 8; j++) step(cu[j]);
       }
-      if (!ok && tid == 0) fail = 1;
+      for (int i = full; i < cn; i++) step(st[i]);
+    } else if (c0 + ENC_CHUNK < n) {
+      fill(c0 + ENC_CHUNK, tid - 64, 192);
     }
     __syncthreads();
   }
   if (tid == 0) {
-    if (fail || cap_b - 4 * k < 8) {
+    if (2LL * n - 4LL * k < 8) {
       atomicMax(&w.err, (int)PK_OVERFLOW);
     } else {
-      out_words[cap_w - 2 - k] = (uint32_t)x;
-      out_words[cap_w - 1 - k] = (uint32_t)(x >> 32);
-      w.dlen = (int)(8 + 4 * k);
-      w.pad = (int)((cap_w - 2 - k) * 4);  // stream start within the slot
+      out_words[cap_w - 2 - k] = (uint32_t)B;
+      out_words[cap_w - 1 - k] = (uint32_t)A;
+      w.dlen = 8 + 4 * k;
+      w.pad = (cap_w - 2 - k) * 4;  // stream start within the slot
     }
   }
 }
@@ -518,56 +539,52 @@ __global__ void pk_headers(const long long* __restrict__ off, const int* __restr
   o[3] = (uint8_t)(r >> 24);
 }
 
-// ---- decode 2: rANS64, one workgroup per window.  cum -> (start, freq, value) in LDS; wave 0
-// runs the state loop from the last value to the first, staging values in LDS chunks that the
-// workgroup then writes out. ----
-constexpr int DEC_CHUNK = 4096;
+// ---- decode 2: rANS64, one workgroup per window.  As in the encoder the launch lasts as long as
+// one wave's serial chain: slot c = x % 4096 names the symbol, x' = freq (x / 4096) + c - start.
+// Every slot's freq and c - start sit in LDS, and the wave-uniform state stays on the vector unit:
+// each trip of a value from the vector to the scalar unit costs ~16 clk and one back into an
+// instruction's lane select or branch as much again, against ~5 clk for a dependent vector
+// instruction and ~48 for the LDS read.  Slots are collected one lane per symbol and turned into
+// values 64 at a time; the stream's words are held 64 at a time in a register as well.
+// 48 windows of up to 512 rows (65,536 steps): 8.14 -> 3.26 ms. ----
 __global__ __launch_bounds__(256) void pk_rans_dec(const uint8_t* __restrict__ in, PkWin* __restrict__ win, int cols,
                                                     float* __restrict__ out) {
-  __shared__ uint32_t cum_sf[RANS_TOTAL];  // start | freq << 16
+  __shared__ uint2 slot[RANS_TOTAL];     // 8 freq, 8 (c - start)
   __shared__ float cum_v[RANS_TOTAL];
-  __shared__ float stage[DEC_CHUNK];
-  __shared__ int st_err;
+  __shared__ uint32_t runs[RANS_TOTAL];  // start | freq << 16 of each symbol
+  __shared__ uint32_t red[4];
   PkWin& w = win[blockIdx.x];
   const int tid = threadIdx.x, n = w.rows * cols, m = w.m;
   // freq 4096 (a single symbol) needs 13 bits next to the 16-bit start: start | freq << 16
   const uint8_t* pairs = in + w.hdr + cols + 2;  // after perm bytes and u16 m
-  __shared__ uint32_t run_start[4097];
+  auto freq = [&](int i) -> uint32_t { return pairs[4 * i + 2] | (pairs[4 * i + 3] << 8); };
   for (int c = tid; c < RANS_TOTAL; c += 256) {
-    cum_sf[c] = 1u << 16;  // slots no symbol covers keep RansDecSymbol::new(0, 1) and 0.0
+    slot[c] = make_uint2(8, 8 * c);  // slots no symbol covers keep RansDecSymbol::new(0, 1) and 0.0
     cum_v[c] = 0.f;
   }
-  if (tid == 0) {
-    st_err = 0;
-    uint32_t cum = 0;
-    for (int i = 0; i < m && i < RANS_TOTAL; i++) {
-      run_start[i] = cum;
-      cum += pairs[4 * i + 2] | (pairs[4 * i + 3] << 8);
-      if (cum > (uint32_t)RANS_TOTAL) st_err = PK_CORRUPT;  // the reference indexes past its tables
-    }
-    if (m > RANS_TOTAL) st_err = PK_CORRUPT;
-  }
-  __syncthreads();
-  if (st_err) {
-    if (tid == 0) atomicMax(&w.err, st_err);
+  // more symbols or a larger total than slots: the reference indexes past its tables
+  const uint32_t total = m > RANS_TOTAL ? RANS_TOTAL + 1u : pk_starts(m, freq, runs, red);
+  if (total > (uint32_t)RANS_TOTAL) {
+    if (tid == 0) atomicMax(&w.err, (int)PK_CORRUPT);
     return;  // uniform
   }
   for (int i = tid; i < m; i += 256) {
-    const uint32_t sym = pairs[4 * i] | (pairs[4 * i + 1] << 8), f = pairs[4 * i + 2] | (pairs[4 * i + 3] << 8);
+    const uint32_t sym = pairs[4 * i] | (pairs[4 * i + 1] << 8), start = runs[i] & 0xffffu, f = runs[i] >> 16;
     float v = 0.f;
     if (sym != 0) {
       const uint32_t q = sym + 1;
       v = (1.0f / 29.0f) * ((q & 1) ? -1.0f : 1.0f) * (float)(q >> 1);
     }
-    const uint32_t start = run_start[i];
     for (uint32_t c = start; c < start + f; c++) {
-      cum_sf[c] = start | (f << 16);
+      slot[c] = make_uint2(8 * f, 8 * (c - start));
       cum_v[c] = v;
     }
   }
   __syncthreads();
+  if (tid >= 64) return;  // wave 0 alone from here: no barrier follows
+  const int lane = tid;
   // The stream, read 4 bytes at a time from any byte offset: two aligned dwords funnel-
-  // shifted (the input buffer carries 16 bytes of padding).  Addresses are wave-uniform.
+  // shifted (the input buffer carries 16 bytes of padding).
   const uint8_t* d = in + w.data;
   const int clen = w.dlen;
   auto word_at = [&](int p) -> uint32_t {
@@ -576,44 +593,70 @@ __global__ __launch_bounds__(256) void pk_rans_dec(const uint8_t* __restrict__ i
     const unsigned long long two = ((unsigned long long)q[1] << 32) | q[0];
     return (uint32_t)(two >> (8 * (a & 3)));
   };
+  // words 64 b .. 64 b + 63 after the state, one per lane; lanes past the stream re-read its end
+  auto words = [&](int b) { return word_at(min(8 + 4 * (64 * b + lane), clen - 4)); };
   float* dst = out + (size_t)w.row0 * cols;
-  unsigned long long x = ((unsigned long long)word_at(4) << 32) | word_at(0);
-  int pos = 8;
+  unsigned long long x = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane(word_at(4)) << 32 |
+                         (uint32_t)__builtin_amdgcn_readfirstlane(word_at(0));
+  asm volatile("" : "+v"(x));  // wave-uniform, but kept on the vector unit: scalar crossings cost more
+  uint32_t wcur = words(0), wnext = words(1);
+  const int avail = (clen - 8) / 4;  // whole words after the state
+  int used = 0;
   bool bad = false;
-  uint32_t next = word_at(min(pos, clen - 4));  // prefetched renormalisation word
-  // decode positions n-1 .. 0 in chunks of DEC_CHUNK (chunk j covers [hi - cn, hi))
-  for (int hi = n; hi > 0; hi -= DEC_CHUNK) {
-    const int cn = min(DEC_CHUNK, hi);
-    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0 && !bad) {
-      // wave 0, wave-uniform state in scalar registers (table entries pass through readfirstlane)
-      for (int i = cn - 1; i >= 0; i--) {
-        const uint32_t c = (uint32_t)(x & (RANS_TOTAL - 1));
-        const uint32_t sf = __builtin_amdgcn_readfirstlane(cum_sf[c]);
-        stage[i] = cum_v[c];
-        x = (unsigned long long)(sf >> 16) * (x >> RANS_BITS) + c - (sf & 0xffffu);
-        if (x < RANS_L) {
-          if (pos + 4 > clen) {
-            bad = true;
-            break;
-          }
-          x = (x << 32) | next;
-          pos += 4;
-          next = word_at(min(pos, clen - 4));
-          if (x < RANS_L) {
-            bad = true;
-            break;
-          }
-        }
+  // e: the entry of x's slot, already requested.  Only two instructions stand between an entry
+  // and the request for the next one: the byte offset of x' % 4096 needs just the low bits of
+  // q = x / 4096 (a 24-bit multiply-add of the entry's factors of 8) and a mask.  x' itself, the
+  // renormalisation test and its branch run while the entry is on its way.
+  auto lookup = [&](uint32_t v8) {
+    return *reinterpret_cast<const uint2*>(reinterpret_cast<const char*>(slot) + (v8 & (8 * RANS_TOTAL - 8)));
+  };
+  uint2 e = lookup((uint32_t)x << 3);
+  auto step = [&]() -> uint32_t {
+    const uint32_t c = (uint32_t)x & (RANS_TOTAL - 1);
+    const unsigned long long q = x >> RANS_BITS;
+    const uint2 next = lookup((uint32_t)__umul24(e.x, (uint32_t)q) + e.y);
+    const uint32_t f = e.x >> 3;
+    const unsigned long long y = (unsigned long long)f * (uint32_t)q + (e.y >> 3);
+    // q < 2^52 and freq < 2^13: the high product fits 24-bit operands
+    typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+    x = __builtin_bit_cast(unsigned long long,
+                           u2v{(uint32_t)y, (uint32_t)(y >> 32) + (uint32_t)__umul24(f, (uint32_t)(q >> 32))});
+    e = next;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(x < RANS_L) != 0, 0)) {  // all lanes alike
+      asm volatile("" : "+v"(e.x), "+v"(e.y));  // used on both sides, so requested before the branch
+      if (used >= avail) bad = true;
+      x = x << 32 | (uint32_t)__builtin_amdgcn_readlane(wcur, used & 63);
+      if ((++used & 63) == 0) {
+        wcur = wnext;
+        wnext = words(used / 64 + 1);
       }
+      if (__builtin_amdgcn_ballot_w64(x < RANS_L)) bad = true;
+      e = lookup((uint32_t)x << 3);
     }
-    if (tid == 0 && bad) st_err = PK_CORRUPT;
-    __syncthreads();
-    for (int i = tid; i < cn; i += 256) dst[hi - cn + i] = stage[i];
-    __syncthreads();
+    return c;
+  };
+  // the j-th symbol decoded is position n - 1 - j
+  int j0 = 0;
+  for (; j0 + 64 <= n && !bad; j0 += 64) {
+    uint32_t slots = 0;
+#pragma unroll
+    for (int j = 0; j < 64; j++) {
+      const uint32_t c = step();
+      slots = lane == j ? c : slots;
+    }
+    dst[n - 1 - j0 - lane] = cum_v[slots];
+  }
+  if (j0 < n && !bad) {
+    uint32_t slots = 0;
+    for (int j = 0; j < n - j0; j++) {
+      const uint32_t c = step();
+      if (lane == j) slots = c;
+    }
+    if (lane < n - j0) dst[n - 1 - j0 - lane] = cum_v[slots];
   }
   if (tid == 0) {
-    if (st_err) atomicMax(&w.err, st_err);
-    w.pad = pos;  // bytes consumed
+    if (bad) atomicMax(&w.err, (int)PK_CORRUPT);
+    w.pad = 8 + 4 * used;  // bytes consumed
   }
 }
 
