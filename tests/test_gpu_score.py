@@ -121,14 +121,59 @@ def test_matmul_argmax_vs_oracle(score, M, N, D, bf16_b):
 
 @pytest.mark.parametrize("bf16_b", [False, True])
 def test_matmul_argmax_many_rows_vs_oracle(score, bf16_b):
-    # M >= 256 x CUs routes to the register-A / LDS-B kernel; 300 columns = 4 full 64-column
-    # chunks + 44, M = 512 x 128 + 37 leaves a partial last workgroup
+    # 300 columns = 4 full 64-column chunks + 44; M = 512 x 128 + 37 leaves a partial last workgroup
     M, N, D = 65573, 300, 128
     print(f"argmax rows M={M} N={N} bf16_b={bf16_b}", flush=True)
     a, b = _data(M, N, D, seed=77)
     got = score.matmul_argmax(a, b, bf16_b=bf16_b)
     assert np.all(got < N)
     assert _check_argmax(a, b, got, bf16_b) >= 0.99 * M
+
+
+# rows x columns around the four tile heights (64, 128, 256 and 512 rows per workgroup on 256 CUs)
+# and around the 64- and 128-column chunks
+@pytest.mark.parametrize("bf16_b", [False, True])
+@pytest.mark.parametrize("M,N", [(1, 2), (63, 64), (65, 129), (16385, 65), (32769, 127), (65537, 63), (131073, 70)])
+def test_matmul_argmax_tiles_vs_oracle(score, M, N, bf16_b):
+    a, b = _data(M, N, 128, seed=M + N)
+    got = score.matmul_argmax(a, b, bf16_b=bf16_b)
+    assert np.all(got < N)
+    assert _check_argmax(a, b, got, bf16_b) >= 0.98 * M
+
+
+# Operands outside the range of the f16 parts take the f32 products: rows and columns of other
+# magnitudes, zeros first, infinities and NaN, in the first chunk or a later one
+@pytest.mark.parametrize("col", [0, 3, 200])
+@pytest.mark.parametrize("what", ["tiny", "huge", "zero", "zero_chunk", "inf", "nan", "rows"])
+def test_matmul_argmax_ranges_vs_oracle(score, what, col):
+    a, b = _data(300, 300, 128, seed=col)
+    with np.errstate(all="ignore"):
+        if what == "tiny":
+            b[col] *= np.float32(1e-6)
+        elif what == "huge":
+            b[col] *= np.float32(1e5)
+        elif what == "zero":
+            b[col] = 0
+        elif what == "zero_chunk":
+            b[:130] = 0
+        elif what == "inf":
+            b[col, 5] = np.inf
+        elif what == "nan":
+            b[col, 7] = np.nan
+        else:
+            a[col % 300] *= np.float32(1e30)
+            a[(col + 1) % 300] *= np.float32(1e-30)
+            a[(col + 2) % 300] = 0
+    got = score.matmul_argmax(a, b)
+    if what in ("inf", "nan"):
+        s = a.astype(np.float64) @ b.astype(np.float64).T
+        s[np.isnan(s)] = -np.inf
+        want = s.argmax(1)
+        top2 = np.sort(s, axis=1)[:, -2:]
+        clear = ~(top2[:, 1] - top2[:, 0] <= 1e-4)
+        np.testing.assert_array_equal(got[clear], want[clear])
+    else:
+        assert _check_argmax(a, b, got, False) >= 0.95 * 300
 
 
 def test_matmul_argmax_exact_ties_first_index(score):

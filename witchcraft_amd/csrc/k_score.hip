@@ -17,6 +17,7 @@
 //   * argmax:   workgroup = 4 waves on 64 rows, looping over N in 256-column chunks; the
 //     running (max, index) per row lives in registers, the 4 waves' results meet in LDS.
 //     Ties resolve to the smallest column index (candle's argmax keeps the first maximum).
+//     128-d rows run on f16 MFMAs with split operands (matmul_argmax_split_kernel).
 #include "common.hpp"
 
 #include <algorithm>
@@ -336,20 +337,63 @@ __global__ __launch_bounds__(256) void matmul_argmax_kernel(const float* __restr
   }
 }
 
-// k-means assignment (src/lib.rs:233-236, 1330) at D = 128 and large M: MFMA-bound.  Each
-// wave owns 32 rows of A, held in registers for the whole run (16 float4 per lane); the 4
-// waves of a workgroup share each 64-column chunk of B through LDS (double-buffered: the
-// next chunk's global loads are issued before this chunk's MFMAs, one barrier per chunk).
-// Global traffic per MFMA is a quarter of the per-wave tile above, which was bound by
-// L2 -> CU bandwidth.  Per row: running (max, first index), as in matmul_argmax_kernel.
+// k-means assignment (src/lib.rs:233-236, 1330) at D = 128: argmax of the f32 products, bound by
+// the matrix cores.  An f32 MFMA runs at 1/16 of the f16 rate, so both operands are split into two
+// f16 parts of a power-of-two multiple (x s = hi + lo + r, |r| <= 2^-23 of x's binade) and a
+// product is hi hi + hi lo + lo hi, each exact in the f32 accumulator: 3 f16 MFMAs for 16 f32
+// ones.  What is dropped (lo lo and the r terms) is at most 2^-21 |a b| per product, without a
+// common sign over the 128 products; the f32 accumulation takes 24 steps where the f32 MFMAs take
+// 32.  (131,072 normal rows x 16,384 normal columns, three seeds: 0, 0 and 2 rows other than in
+// 64 bits, against 1, 0 and 2 on f32 MFMAs.)
+//  * Rows of A: each scaled by its own power of two (an argmax over the row does not change) and
+//    held in registers for the whole run, 32 RBL rows per wave on 32x32x16 MFMAs.
+//  * Columns of B: 64 or 128 at a time through double-buffered LDS, split once per workgroup on
+//    the way in, all by one power of two set from the first columns.  A column must then stay
+//    inside f16's precise range: largest |b s| in [2^3, 2^15], or all zeros.
+//  * A row or column outside those ranges, infinite or NaN makes the workgroup redo its rows on
+//    f32 MFMAs (argmax_rows_f32), so such inputs give what they gave before.
+// The 8 waves of a workgroup hold 8 / WN row groups; the WN waves of a group take 1 / WN of a
+// chunk's columns each, for inputs with too few rows to fill the chip.
+// 131,072 x 16,384: 5.03 ms on f32 MFMAs (109 TFLOP/s) -> 1.28-1.40 ms (390-430); 4,096 x 4,096:
+// 228 -> 76 us.  Counters on an earlier form of the loop: MFMA busy 56% at a 1.7 GHz clock, the
+// rest vector work (splitting B, the running maxima).
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ uint32_t float_exp(float v) { return (__float_as_uint(v) >> 23) & 0xffu; }
+__device__ __forceinline__ float pow2_bits(uint32_t biased) { return __uint_as_float(biased << 23); }
+__device__ __forceinline__ float max4abs(float4 v) {
+  return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+// Not finite (fmaxf drops NaNs, so the largest magnitude alone does not tell).
+__device__ __forceinline__ bool odd4(float4 v) {
+  const float z = (v.x - v.x) + (v.y - v.y) + (v.z - v.z) + (v.w - v.w);
+  return !(z == 0.f);
+}
+// Largest of the 32 lanes of a wave half.
+__device__ __forceinline__ float max32(float v) {
+#define T5K_ROR(n) v = fmaxf(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + (n), 0xf, 0xf, false)))
+  T5K_ROR(8);
+  T5K_ROR(4);
+  T5K_ROR(2);
+  T5K_ROR(1);
+#undef T5K_ROR
+  return max_xor16(v);
+}
+// s x = hi + lo, each rounded to nearest f16
+__device__ __forceinline__ void split_f16(float x, float s, _Float16& hi, _Float16& lo) {
+  hi = (_Float16)(x * s);
+  lo = (_Float16)__builtin_fmaf(x, s, -(float)hi);
+}
+
+// 256 rows from wg_r0 (8 waves of 32) on f32 MFMAs: A in registers, 64-column chunks of B through
+// double-buffered LDS (Bs, 2 x 64 x 33 float4).
+constexpr int ARG_F32_LDS = 2 * 64 * 33;
 template <bool BF16B>
-__global__ __launch_bounds__(256, 2) void matmul_argmax_rows_kernel(const float* __restrict__ A,
-                                                                    const float* __restrict__ B,
-                                                                    uint32_t* __restrict__ out, int M, int N) {
+__device__ __forceinline__ void argmax_rows_f32(const float* __restrict__ A, const float* __restrict__ B,
+                                             uint32_t* __restrict__ out, int M, int N, int wg_r0, float4* Bs) {
   constexpr int D = 128, KB = D / 16, BS = D / 4 + 1, RB = 2;  // LDS row stride: 33 float4
-  __shared__ float4 Bs[2][64 * BS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
-  const int r0 = blockIdx.x * (64 * RB) + wave * (16 * RB);
+  const int r0 = wg_r0 + wave * (16 * RB);
   // A fragments: row r0 + 16 mb + lr, K slice 16 kb + 4 lg; rows past M repeat row M - 1
   // (their results are not stored)
   float4 a[KB][4];
@@ -359,21 +403,21 @@ __global__ __launch_bounds__(256, 2) void matmul_argmax_rows_kernel(const float*
 #pragma unroll
     for (int kb = 0; kb < KB; kb++) a[kb][mb] = ldg4(p + 16 * kb);
   }
-  // chunk loader: thread tid moves float4 q = tid + 256 j (j < 8) of the 64 x 32 float4 chunk;
+  // chunk loader: thread tid moves float4 q = tid + 512 j (j < 4) of the 64 x 32 float4 chunk;
   // columns past N repeat column N - 1 (masked out of the argmax)
-  float4 st[8];
+  float4 st[4];
   auto gload = [&](int n0) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int q = tid + 256 * j, c = q >> 5, k4 = q & 31;
+    for (int j = 0; j < 4; j++) {
+      const int q = tid + 512 * j, c = q >> 5, k4 = q & 31;
       st[j] = ldg4(B + (size_t)min(n0 + c, N - 1) * D + 4 * k4);
     }
   };
   auto lstore = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int q = tid + 256 * j, c = q >> 5, k4 = q & 31;
-      Bs[buf][c * BS + k4] = BF16B ? trunc_bf16(st[j]) : st[j];
+    for (int j = 0; j < 4; j++) {
+      const int q = tid + 512 * j, c = q >> 5, k4 = q & 31;
+      Bs[buf * 64 * BS + c * BS + k4] = BF16B ? trunc_bf16(st[j]) : st[j];
     }
   };
   float bv[RB];
@@ -399,7 +443,7 @@ __global__ __launch_bounds__(256, 2) void matmul_argmax_rows_kernel(const float*
     for (int kb = 0; kb < KB; kb++) {
       float4 b[4];
 #pragma unroll
-      for (int nb = 0; nb < 4; nb++) b[nb] = Bs[buf][(16 * nb + lr) * BS + 4 * kb + lg];
+      for (int nb = 0; nb < 4; nb++) b[nb] = Bs[buf * 64 * BS + (16 * nb + lr) * BS + 4 * kb + lg];
       mfma_4x4<RB>(a[kb], b, acc);
     }
 #pragma unroll
@@ -431,6 +475,224 @@ __global__ __launch_bounds__(256, 2) void matmul_argmax_rows_kernel(const float*
     for (int mb = 0; mb < RB; mb++) {
       const int r = r0 + 16 * mb + lr;
       if (r < M) out[r] = (uint32_t)bi[mb];
+    }
+}
+
+template <bool BF16B, int RBL, int WN>
+__global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float* __restrict__ A,
+                                                                     const float* __restrict__ B,
+                                                                     uint32_t* __restrict__ out, int M, int N) {
+  constexpr int D = 128, KS = D / 16, PARTS = BF16B ? 1 : 2;  // a truncated b s is one f16
+  constexpr int COLS = WN == 4 ? 128 : 64, CB = COLS / 32 / WN, NL = COLS / 16;
+  constexpr int PART = COLS * 16;  // h8 per part of a chunk: COLS columns x 16 chunks of 8 k
+  constexpr int LDS4 = 2 * PARTS * PART > ARG_F32_LDS ? 2 * PARTS * PART : ARG_F32_LDS;
+  __shared__ float4 lds[LDS4];  // chunks [2][PARTS][PART] h8, or argmax_rows_f32's
+  __shared__ float red[8];
+  __shared__ int redo[2];  // by barrier parity: a flag is rewritten only after every thread has read it
+  h8* Bs = reinterpret_cast<h8*>(lds);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, lr = lane & 31, lg = lane >> 5;
+  constexpr int wg_rows = 32 * RBL * (8 / WN);
+  const int wg_r0 = blockIdx.x * wg_rows, r0 = wg_r0 + (wave / WN) * 32 * RBL, cb0 = (wave % WN) * CB;
+  bool bad = false;
+  // thread tid moves the float4 k4 of columns c0 + 16 j (j < NL) of a chunk, 32 lanes to a column;
+  // columns past N repeat column N - 1, which then ties with itself at a larger index
+  const int c0 = tid >> 5, k4 = tid & 31;
+  float4 st[NL];
+  auto gload = [&](int n0) {  // also past the last chunk: unconditional, so nothing waits for it early
+#pragma unroll
+    for (int j = 0; j < NL; j++)
+      st[j] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(B) +
+                                               ((uint32_t)min(n0 + c0 + 16 * j, N - 1) * (4u * D) + 16u * k4));
+  };
+  gload(0);
+  {  // one power of two for every column: the first chunk's largest magnitude comes to [2^12, 2^13)
+    float m = 0.f;
+#pragma unroll
+    for (int j = 0; j < NL; j++) m = fmaxf(m, max4abs(BF16B ? trunc_bf16(st[j]) : st[j]));
+    m = max_xor32(max32(m));
+    if (lane == 0) red[wave] = m;
+    if (tid == 0) redo[0] = redo[1] = 0;
+  }
+  __syncthreads();
+  float bmax = red[0];
+#pragma unroll
+  for (int i = 1; i < 8; i++) bmax = fmaxf(bmax, red[i]);
+  const uint32_t be = float_exp(bmax);
+  if (be < 40 || be > 250) bad = true;  // zeros, tiny, huge, infinite
+  const float bs = pow2_bits(bad ? 127 : 127 + 12 + 127 - be);
+  // 16-byte chunk k / 8 of column c sits at chunk (k / 8) ^ (c % 16): the operand reads below (32
+  // columns x one chunk) and these stores (one column, 16 chunks) hit every bank once
+  const int at0 = (c0 * 16 + ((k4 >> 1) ^ c0)) * 2 + (k4 & 1);
+  auto lstore = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < NL; j++) {
+      const float4 v = BF16B ? trunc_bf16(st[j]) : st[j];
+      // largest magnitude as an integer: infinities and NaNs compare above every finite value
+      const uint32_t u = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
+                             max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
+      const float m = __uint_as_float(u) * bs;
+      // a column is a wave half: some lane reaches 2^3 or every lane is zero
+      const unsigned long long big = __builtin_amdgcn_ballot_w64(m >= 8.f), any = __builtin_amdgcn_ballot_w64(u != 0);
+      bad |= !(m <= 32768.f) || ((uint32_t)big == 0 && (uint32_t)any != 0) || (big >> 32 == 0 && any >> 32 != 0);
+      h4 hi, lo;
+      _Float16 h, l;
+      split_f16(v.x, bs, h, l); hi[0] = h; lo[0] = l;
+      split_f16(v.y, bs, h, l); hi[1] = h; lo[1] = l;
+      split_f16(v.z, bs, h, l); hi[2] = h; lo[2] = l;
+      split_f16(v.w, bs, h, l); hi[3] = h; lo[3] = l;
+      h4* dst = reinterpret_cast<h4*>(Bs + buf * PARTS * PART) + at0 + j * (16 * 16 * 2);
+      dst[0] = hi;
+      if (PARTS == 2) dst[PART * 2] = lo;
+    }
+  };
+  lstore(0);
+  gload(COLS);
+  // A operand of K step ks: row r0 + 32 rb + lr, k = 16 ks + 8 lg .. +7; rows past M repeat row M - 1
+  h8 ah[RBL][KS], al[RBL][KS];
+#pragma unroll
+  for (int rb = 0; rb < RBL; rb++) {
+    const float* p = A + (size_t)min(r0 + 32 * rb + lr, M - 1) * D + 8 * lg;
+    float4 v[2 * KS];
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < 2 * KS; i++) {
+      v[i] = ldg4(p + 16 * (i >> 1) + 4 * (i & 1));
+      m = fmaxf(m, max4abs(v[i]));
+      bad |= odd4(v[i]);
+    }
+    m = max_xor32(m);
+    const uint32_t e = float_exp(m);
+    bad |= e > 250 || (e < 40 && m != 0.f);
+    const float as = pow2_bits(e > 250 || e < 40 ? 127 : 127 + 12 + 127 - e);
+#pragma unroll
+    for (int i = 0; i < 2 * KS; i++) {
+      const float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        _Float16 h, l;
+        split_f16(x[j], as, h, l);
+        ah[rb][i >> 1][4 * (i & 1) + j] = h;
+        al[rb][i >> 1][4 * (i & 1) + j] = l;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float bv[RBL];
+  int bi[RBL];
+#pragma unroll
+  for (int rb = 0; rb < RBL; rb++) {
+    bv[rb] = -INFINITY;
+    bi[rb] = 0;
+  }
+  if (bad) redo[0] = 1;
+  __syncthreads();
+  auto multiply = [&](int buf, int n0) {
+#pragma unroll
+    for (int cb = 0; cb < CB; cb++) {
+      f16v acc[RBL];
+#pragma unroll
+      for (int rb = 0; rb < RBL; rb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[rb][i] = 0.f;
+      const h8* bp = Bs + buf * PARTS * PART + (32 * (cb0 + cb) + lr) * 16;
+      // each step's operands are read from LDS one step (3 RBL MFMAs) ahead
+      h8 bh[2], bl[2];
+      auto read = [&](int ks) {
+        const int at = (2 * ks + lg) ^ (lr & 15);
+        bh[ks & 1] = bp[at];
+        if (PARTS == 2) bl[ks & 1] = bp[PART + at];
+      };
+      read(0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) {
+        if (ks + 1 < KS) read(ks + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (PARTS == 2)
+#pragma unroll
+          for (int rb = 0; rb < RBL; rb++)
+            acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl[ks & 1], ah[rb][ks], acc[rb], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < RBL; rb++)
+          acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh[ks & 1], al[rb][ks], acc[rb], 0, 0, 0);
+#pragma unroll
+        for (int rb = 0; rb < RBL; rb++)
+          acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh[ks & 1], ah[rb][ks], acc[rb], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // lane: row lr of the block, columns 8 (i / 4) + 4 lg + i % 4 of the 32, ascending in i, so
+      // the first of equal scores is kept by "greater" over chunks and a descending search inside
+#pragma unroll
+      for (int rb = 0; rb < RBL; rb++) {
+        float m = acc[rb][0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) m = fmaxf(m, acc[rb][i]);
+        if (m > bv[rb]) {
+          int ix = 15;
+#pragma unroll
+          for (int i = 14; i >= 0; i--) ix = acc[rb][i] == m ? i : ix;
+          bi[rb] = n0 + 32 * (cb0 + cb) + 8 * (ix >> 2) + 4 * lg + (ix & 3);
+          bv[rb] = m;
+        }
+      }
+    }
+  };
+  // Chunk ch + 1 is split into the other buffer while chunk ch is multiplied, by the first wave of
+  // each SIMD (waves 0-3) before its products and by the second after, so one wave's vector work
+  // runs beside the other's MFMAs.
+  const int nchunks = (N + COLS - 1) / COLS;
+  bool f32 = redo[0];  // workgroup-uniform
+  for (int ch = 0; ch < nchunks && !f32; ch++) {
+    const int buf = ch & 1;
+    if (wave < 4) {
+      lstore(buf ^ 1);
+      gload((ch + 2) * COLS);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    multiply(buf, ch * COLS);
+    if (wave >= 4) {
+      lstore(buf ^ 1);
+      gload((ch + 2) * COLS);
+    }
+    if (bad) redo[(ch + 1) & 1] = 1;
+    __syncthreads();
+    f32 = redo[(ch + 1) & 1];
+  }
+  if (f32) {
+    for (int r = wg_r0; r < min(wg_r0 + wg_rows, M); r += 256) {
+      __syncthreads();
+      argmax_rows_f32<BF16B>(A, B, out, min(M, wg_r0 + wg_rows), N, r, lds);
+    }
+    return;
+  }
+  // the two lanes, and the WN waves, that hold parts of a row
+#pragma unroll
+  for (int rb = 0; rb < RBL; rb++) {
+    const float w = __shfl_xor(bv[rb], 32);
+    const int j = __shfl_xor(bi[rb], 32);
+    amax_merge(bv[rb], bi[rb], w, j);
+  }
+  if constexpr (WN > 1) {  // the loop ended with a barrier: the chunks are no longer read
+    float* sv = reinterpret_cast<float*>(lds);
+    int* si = reinterpret_cast<int*>(sv + 8 * 32 * RBL);
+#pragma unroll
+    for (int rb = 0; rb < RBL; rb++)
+      if (lg == 0) {
+        sv[(wave * RBL + rb) * 32 + lr] = bv[rb];
+        si[(wave * RBL + rb) * 32 + lr] = bi[rb];
+      }
+    __syncthreads();
+    if (wave % WN) return;
+#pragma unroll
+    for (int rb = 0; rb < RBL; rb++)
+      for (int w = 1; w < WN; w++)
+        amax_merge(bv[rb], bi[rb], sv[((wave + w) * RBL + rb) * 32 + lr], si[((wave + w) * RBL + rb) * 32 + lr]);
+  }
+  if (lg == 0)
+#pragma unroll
+    for (int rb = 0; rb < RBL; rb++) {
+      const int r = r0 + 32 * rb + lr;
+      if (r < M) out[r] = (uint32_t)bi[rb];
     }
 }
 
@@ -500,13 +762,38 @@ hipError_t launch_matmul_argmax(const float* A, const float* B, uint32_t* out, i
   if (M <= 0) return hipSuccess;
   if (N <= 0 || D < 0) return hipErrorInvalidValue;
   const bool vec = D % 4 == 0 && aligned16(A) && aligned16(B);
-  if (vec && D == 128 && M >= 256L * num_cus()) {
-    // enough rows for two 128-row workgroups per CU: the register-A / LDS-B kernel
-    const dim3 g((M + 127) / 128);
-    if (bf16_b)
-      hipLaunchKernelGGL((matmul_argmax_rows_kernel<true>), g, dim3(256), 0, s, A, B, out, M, N);
-    else
-      hipLaunchKernelGGL((matmul_argmax_rows_kernel<false>), g, dim3(256), 0, s, A, B, out, M, N);
+  if (vec && D == 128 && N < (1 << 23)) {  // byte offsets of B fit 32 bits
+    // Rows per workgroup (one workgroup per CU at a time): a shorter tile re-splits B more often per
+    // row but fills the chip with fewer rows.  Times of one round over 4,096 columns: 512 rows 279
+    // us, 256 rows 195, 128 rows 110, 64 rows 80; the least rounds x time is taken (16,384 x 4,096:
+    // 80 us on 64 rows, 97 on 128, 166 on 256, 258 on 512, 233 on the f32 kernel below).
+    const long cus = num_cus();
+    const double cost[4] = {279, 195, 110, 80};
+    int v = 0;
+    double best = 1e30;
+    for (int i = 0; i < 4; i++) {
+      const long rows = 512 >> i, wgs = (M + rows - 1) / rows;
+      const double t = (double)((wgs + cus - 1) / cus) * cost[i];
+      if (t < best) {
+        best = t;
+        v = i;
+      }
+    }
+#define T5K_AMS(RBL, WN)                                                                                          \
+  do {                                                                                                            \
+    const dim3 g((M + 256 * RBL / WN - 1) / (256 * RBL / WN));                                                    \
+    if (bf16_b)                                                                                                   \
+      hipLaunchKernelGGL((matmul_argmax_split_kernel<true, RBL, WN>), g, dim3(512), 0, s, A, B, out, M, N);         \
+    else                                                                                                          \
+      hipLaunchKernelGGL((matmul_argmax_split_kernel<false, RBL, WN>), g, dim3(512), 0, s, A, B, out, M, N);        \
+  } while (0)
+    switch (v) {
+      case 0: T5K_AMS(2, 1); break;
+      case 1: T5K_AMS(2, 2); break;
+      case 2: T5K_AMS(1, 2); break;
+      default: T5K_AMS(1, 4); break;
+    }
+#undef T5K_AMS
     return hipGetLastError();
   }
   const dim3 grid((M + 63) / 64);
