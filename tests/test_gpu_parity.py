@@ -764,6 +764,30 @@ def test_tile_width_does_not_change_bits(enc_mod, xtr):
             h.close()
 
 
+# token counts over which the planner goes through every form and tile, each a few tokens past or
+# short of whole tiles
+@pytest.mark.parametrize("layout", ["q4k", "hybrid"])
+def test_gemm_forms_are_bit_identical(enc_mod, xtr, layout):
+    """The ring and direct GEMM forms take K in one order: the planner's choice at every size gives
+    the bits of 256 x 128 direct tiles, and a small batch those of 64 x 128 ones."""
+    cfg, img, gpu, _ = xtr
+    if layout == "hybrid":
+        img = synth.make_model(cfg, seed=3, layout="hybrid")
+        gpu = enc_mod.T5EncoderModel.from_gguf(img, cfg)
+    hs = [_handle_with_env(enc_mod, img, cfg, T5H_GEMM_TAIL=t) for t in ("0", "1")]
+    try:
+        for T in (65, 127, 161, 255, 300, 513, 700, 1100, 1700, 2100, 3300, 4700, 6300, 9001, 13000):
+            cu = np.unique(np.r_[0:T:500, T]).astype(np.int32)
+            ids = np.random.default_rng(T).integers(1, cfg["vocab_size"], size=T).astype(np.uint32)
+            got, _ = gpu.encode_packed(ids, cu)
+            for h in hs[:1 if T > 2100 else 2]:
+                ref, _ = h.encode_packed(ids, cu)
+                assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), (layout, T)
+    finally:
+        for h in hs:
+            h.close()
+
+
 @pytest.mark.parametrize("lens", [[5, 11, 16], [1, 1, 1, 29], [0, 7, 0, 9], [31], [16, 16]])
 def test_small_multi_sequence_batches_vs_oracle(xtr, lens):
     """Query-sized batches (the small-token GEMV path) holding several sequences, empty ones

@@ -67,6 +67,8 @@ struct GemmArgs {
   int lda;            // unused (A's row length is K)
   const void* W0;  // [N][K] weights (Q4_K blocks row-major along K, or f16)
   const void* W1;  // second weight for EPI_GATED
+  const _Float16* T0;  // W0 and W1 as launch_tile_weights lays them out (batched GEMM)
+  const _Float16* T1;
   int M, N, K;     // N counts output columns (per weight for EPI_GATED)
   void* out;
   int ldo;
@@ -143,13 +145,6 @@ struct AttnArgs {
 
 // Device-side helpers ---------------------------------------------------------
 
-// LDS tiles of f16 with 64-half rows, unpadded, where 16-byte chunk c of row r is stored at
-// chunk c ^ (r & 7): a read of 16 rows x one chunk (ds_read_b128) and a transposed read of 16
-// rows x 32 bytes (ds_read_b64_tr_b16) each hit every bank once (measured with probe kernels).
-__device__ __forceinline__ int swz64(int row, int col) {
-  return row * 64 + ((((col >> 3) ^ row) & 7) << 3) + (col & 7);
-}
-
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t bits16) {
   _Float16 h;
   uint16_t b = (uint16_t)bits16;
@@ -205,20 +200,31 @@ namespace t5k {
 hipError_t launch_q4k_dequant(const void* blocks, size_t nblk, float* out, hipStream_t s);
 // Q4_K -> f32 (exact) -> bf16 truncation -> f16, [nblk * 256] in block order.
 hipError_t launch_q4k_dequant_bf16_f16(const void* blocks, size_t nblk, _Float16* out, hipStream_t s);
-// Tile plan of one batched GEMM launch: full tiles of 64*mw token rows x bn weight rows
-// cover rows [0, m_main); thin tiles of 16*tail_mb rows per math wave cover [m_main, M)
-// (tail_mb = 0: full tiles everywhere).
-// mb: 16-token row blocks per math wave in the full tiles (4, or 3 with mw = 4).
-struct GemmPlan {
-  int mw = 4, bn = 128, m_main = 0, tail_mb = 0, mb = 4;
+// Kernel and tile (tokens x weight rows) of one batched GEMM launch (k_gemm.hip).  gemm_plan chooses
+// among the first GEMM_AUTO_VARIANTS; the rest serve the tuning knobs and tests.
+enum GemmVariant : int {
+  GEMM_RING_32X64,
+  GEMM_RING_64X64,
+  GEMM_RING_128X64,
+  GEMM_RING_128X128,    // four steps deep, one workgroup per CU
+  GEMM_RING_128X128_2,  // two steps deep, two workgroups per CU
+  GEMM_128X128,
+  GEMM_192X128,
+  GEMM_256X128,
+  GEMM_AUTO_VARIANTS,
+  GEMM_64X128 = GEMM_AUTO_VARIANTS,
+  GEMM_256X64,
 };
-GemmPlan gemm_plan(int M, int n_rows, int cus, int mw_override, int bn_override, int tail_override,
-                   int mb_override = 0);
-hipError_t launch_gemm(int epi, int wfmt, const GemmPlan& plan, const GemmArgs& a, hipStream_t s);
+struct GemmPlan {
+  int variant = GEMM_256X128;
+};
+GemmPlan gemm_plan(int epi, int M, int n_rows, int K, int cus);
+hipError_t launch_gemm(int epi, const GemmPlan& plan, const GemmArgs& a, hipStream_t s);
+// The weights as launch_gemm reads them: f16 in operand order (tiled_index), [N][K] values.
+hipError_t launch_tile_weights(const void* w, int wfmt, int N, int K, _Float16* out, hipStream_t s);
 // Small-M variant (M <= GEMV_MAX_M tokens), same arguments and results.
 constexpr int GEMV_MAX_M = 64;
 hipError_t launch_gemv(int epi, int wfmt, const GemmArgs& a, hipStream_t s);
-void gemm_pick_tile(int M, int n_rows, int cus, int& mw, int& bn);
 hipError_t launch_attention(const AttnArgs& a, int n_work, int dkv, hipStream_t s);
 // With rec set, also the first block's T5LayerNorm (weight gamma) in record mode into xn / rec,
 // as launch_rmsnorm's record mode (D <= 1024); rec_stride 16 (batched GEMMs) or 64 (GEMV).
@@ -279,13 +285,18 @@ hipError_t launch_q8k_quantize(const float* x, const float* gamma, float eps, in
                                hipStream_t s, int8_t* xq = nullptr, float* d8 = nullptr, _Float16* bsop = nullptr);
 hipError_t launch_q8k_operands(const uint8_t* blocks, int T, int D, int8_t* xq, float* d8, _Float16* bsop,
                                hipStream_t s);
-// Q4_K weights x Q8_K activations on the matrix cores (k_gemm.hip): per K block of 256, the int8
+// Q4_K weights x Q8_K activations on the matrix cores (k_hybrid.hip): per K block of 256, the int8
 // planes (sc >> 3) q4 and (sc & 7) q4 against int8 q8 sum the block's integers exactly in int32
 // (8 hi + lo); the block then adds d4 d8 * sum - dmin4 d8 * (mins . bsums) in f32.  epi:
 // EPI_GATED (gelu_pade(W0) * W1 into the f16 operand, operand order) or EPI_F32.  Q4_K weights, bn = 64, K <= 1024.
-GemmPlan gemm_plan_hybrid(int M, int n_rows, int cus);
+// Full tiles for rows [0, m_main), thin tiles of 16 tail_mb rows per math wave for the rest
+// (tail_mb = 0: full tiles everywhere).
+struct HybridPlan {
+  int m_main = 0, tail_mb = 0;
+};
+HybridPlan gemm_plan_hybrid(int M, int n_rows, int cus);
 // Rows of the A operand, d8 and bsop a hybrid launch over M tokens may read (its full tiles
 // round M up to the tile height): the buffers must hold at least this many.
 int gemm_hybrid_rows(int M);
-hipError_t launch_gemm_hybrid(int epi, const GemmPlan& plan, const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_hybrid(int epi, const HybridPlan& plan, const GemmArgs& a, hipStream_t s);
 }  // namespace t5k

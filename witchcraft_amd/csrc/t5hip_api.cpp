@@ -95,6 +95,7 @@ struct Linear {
   int fmt = WF_Q4K;
   size_t off = 0;         // byte offset in the weight arena
   const void* w = nullptr;  // device pointer (set after upload)
+  const _Float16* t = nullptr;  // the f16 operand of the batched GEMMs, laid out by build_tiled
   // F32/F16 dense weights also keep f16(bf16_trunc(w)) [N][K] for T5H_NUMERICS_HYBRID_BF16
   // (the source values are only borrowed during t5h_create): arena offset, device pointer.
   bool has_bf = false;
@@ -152,6 +153,7 @@ struct ReplayRec {
   int epi = 0, wfmt = 0, n = 0;
   GemmArgs ga{};
   t5k::GemmPlan plan{};
+  t5k::HybridPlan hplan{};
   AttnArgs aa{};
   // embed / rownorm / rmsnorm
   const uint32_t* ids = nullptr;
@@ -210,14 +212,12 @@ struct t5h_model {
   hipStream_t stream = nullptr;
   int inner = 0;
   int cus = 256;          // compute units of the device
-  int gemm_mw_override = 0;  // T5H_GEMM_MW / T5H_GEMM_BN tuning knobs (0 = heuristic)
+  bool gemv_off = false;      // T5H_GEMM_MW=2/4/8: the batched GEMM at every token count
   bool batched_only = false;  // route every linear through the batched GEMM (t5h_ffn_block mode 1)
-  int gemm_bn_override = 0;
-  int gemm_mb_override = 0;  // T5H_GEMM_MB: 3 / 4 row blocks per math wave in full tiles (0 = choose)
-  int gemm_tail_override = -1;  // T5H_GEMM_TAIL: -1 = choose, 0 = full tiles only, 1 / 2 = thin tail, 3 / 4 = all thin
+  int gemm_variant = -1;      // batched GEMM form and tile for every launch (T5H_GEMM_* knobs; -1 = gemm_plan)
   bool fold_norm_off = false;   // T5H_FOLD_NORM=0: standalone RMSNorm launches on the batched path
   int ffn_chunk = 0;            // T5H_FFN_CHUNK=<tokens, multiple of 512>: FFN in token chunks
-  bool gated_mw8 = false;       // T5H_GATED_MW8=1: gated FFN on 8 math waves of 32 tokens
+  bool gated_mw8 = false;       // T5H_GATED_MW8=1: gated FFN on workgroups of 8 waves of 32 tokens
   // T5H_FFN_FUSED=<tokens>: batches (lane parts) of at least that many tokens run the gated FFN
   // as one launch (k_ffn.hip), bit-identical to the two launches and measured slower; 0 = off.
   int ffn_fused_min = 0;
@@ -241,6 +241,9 @@ struct t5h_model {
   // first switch to that mode.
   std::vector<Layer> layers_bf;
   void* bfw = nullptr;
+  // The batched GEMMs' f16 operands (Linear::t) of `layers` and proj, and of layers_bf.
+  void* tw = nullptr;
+  void* twb = nullptr;
   Linear proj;
 
   // ---- workspace ----
@@ -312,6 +315,8 @@ struct t5h_model {
     if (ws) (void)hipFree(ws);
     if (ew) (void)hipFree(ew);
     if (bfw) (void)hipFree(bfw);
+    if (tw) (void)hipFree(tw);
+    if (twb) (void)hipFree(twb);
     if (arena) (void)hipFree(arena);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -585,7 +590,7 @@ void resolve_timings(t5h_model* m) {
 // Small token counts run the GEMV kernels (unless a tuning override or t5h_ffn_block mode 1
 // forces the batched GEMM).
 bool use_gemv(const t5h_model* m, int M) {
-  return M <= t5k::GEMV_MAX_M && !m->gemm_mw_override && !m->batched_only;
+  return M <= t5k::GEMV_MAX_M && !m->gemv_off && !m->batched_only;
 }
 
 // A T5LayerNorm folded into the batched GEMMs around it (GemmArgs::rec): a consumer passes
@@ -614,6 +619,25 @@ bool hybrid_numerics(const t5h_model* m) { return m->numerics != T5H_NUMERICS_DE
 // The weights block l runs with under the current numerics.
 const Layer& layer_w(const t5h_model* m, int l) {
   return m->numerics == T5H_NUMERICS_HYBRID_BF16 ? m->layers_bf[l] : m->layers[l];
+}
+
+// Lays the given linears out for the batched GEMMs (Linear::t) in one allocation.  Asynchronous on
+// the handle's stream.
+int build_tiled(t5h_model* m, const std::vector<Linear*>& ls, void** buf) {
+  size_t need = 0;
+  for (const Linear* L : ls) need += align256((size_t)L->N * L->K * 2);
+  if (hipMalloc(buf, need) != hipSuccess) {
+    *buf = nullptr;
+    return fail(T5H_ERR_NOMEM, "weight operand allocation of " + std::to_string(need) + " bytes failed");
+  }
+  size_t off = 0;
+  for (Linear* L : ls) {
+    _Float16* dst = (_Float16*)((uint8_t*)*buf + off);
+    HIP_OK(t5k::launch_tile_weights(L->w, L->fmt, L->N, L->K, dst, m->stream));
+    L->t = dst;
+    off += align256((size_t)L->N * L->K * 2);
+  }
+  return T5H_OK;
 }
 
 // The one-launch gated FFN (k_ffn.hip) for this layer and batch: batched path, default numerics,
@@ -661,7 +685,7 @@ int hybrid_linear(t5h_model* m, int kind, const float* ln, const Linear& W0, con
   a.d8 = d8;
   a.bsop = bs;
   const int epi = W1 ? EPI_GATED : EPI_F32;
-  const t5k::GemmPlan plan = t5k::gemm_plan_hybrid(T, W0.N * (W1 ? 2 : 1), m->cus);
+  const t5k::HybridPlan plan = t5k::gemm_plan_hybrid(T, W0.N * (W1 ? 2 : 1), m->cus);
   HIP_OK(t5k::launch_gemm_hybrid(epi, plan, a, m->stream));
   if (m->prof) {
     ReplayRec& r = m->replay[kind];
@@ -676,7 +700,7 @@ int hybrid_linear(t5h_model* m, int kind, const float* ln, const Linear& W0, con
     r.hbs = bs;
     r.epi = epi;
     r.ga = a;
-    r.plan = plan;
+    r.hplan = plan;
   }
   return T5H_OK;
 }
@@ -707,7 +731,8 @@ int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, con
   const double flops = 2.0 * M * W.N * W.K * mats;
   const double out_bytes = (epi == EPI_F32 || epi == EPI_RESID ? 4.0 : 2.0) * M * W.N *
                            (epi == EPI_RESID ? 2.0 : 1.0);
-  const double bytes = W.bytes() * mats + 2.0 * M * W.K + out_bytes;
+  const double w_bytes = use_gemv(m, M) ? (double)W.bytes() : 2.0 * W.N * W.K;  // Q4_K, or the f16 operand
+  const double bytes = w_bytes * mats + 2.0 * M * W.K + out_bytes;
   Timed t(m, kind, flops, bytes);
   if (nl) {
     if (norm_w) return fail(T5H_ERR_INVALID, "internal: fused and folded norm requested together");
@@ -734,16 +759,12 @@ int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, con
     return T5H_OK;
   }
   if (norm_w) return fail(T5H_ERR_INVALID, "internal: fused norm requested on the batched GEMM path");
-  t5k::GemmPlan plan = t5k::gemm_plan(M, W.N * (W1 ? 2 : 1), m->cus, m->gemm_mw_override, m->gemm_bn_override,
-                                      m->gemm_tail_override, m->gemm_mb_override);
-  if (epi == EPI_GATED && m->gated_mw8 && W.fmt == WF_Q4K && W.N % 64 == 0) {
-    plan.mw = 8;  // 256-token tiles of 8 math waves x 32 tokens, 128 weight rows
-    plan.mb = 2;
-    plan.bn = 128;
-    plan.m_main = M;
-    plan.tail_mb = 0;
-  }
-  HIP_OK(t5k::launch_gemm(epi, W.fmt, plan, a, m->stream));
+  a.T0 = W.t;
+  a.T1 = W1 ? W1->t : nullptr;
+  t5k::GemmPlan plan = t5k::gemm_plan(epi, M, W.N * (W1 ? 2 : 1), W.K, m->cus);
+  if (m->gemm_variant >= 0) plan.variant = m->gemm_variant;
+  else if (epi == EPI_GATED && m->gated_mw8) plan.variant = t5k::GEMM_RING_128X128;  // 8 waves of 32 tokens
+  HIP_OK(t5k::launch_gemm(epi, plan, a, m->stream));
   if (m->prof) {
     ReplayRec& r = m->replay[kind];
     r.type = ReplayRec::GEMM;
@@ -1508,19 +1529,22 @@ int create_impl(const void* gguf, size_t len, const t5h_config* cfg, int hip_dev
   m->cus = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
   if (const char* e = getenv("T5H_GEMM_MW")) {
     const int v = atoi(e);
-    if (v == 2 || v == 4 || v == 8) m->gemm_mw_override = v;
+    m->gemv_off = v == 2 || v == 4 || v == 8;
   }
+  // One direct tile for every batched launch: T5H_GEMM_BN=64/128 weight rows, T5H_GEMM_TAIL=0..4 and
+  // T5H_GEMM_MB=3/4 its height (0 and MB 4: 256 tokens, 1 and 3: 64, 2 and 4: 128, MB 3: 192).
   if (const char* e = getenv("T5H_GEMM_BN")) {
     const int v = atoi(e);
-    if (v == 64 || v == 128) m->gemm_bn_override = v;
-  }
-  if (const char* e = getenv("T5H_GEMM_MB")) {
-    const int v = atoi(e);
-    if (v == 3 || v == 4) m->gemm_mb_override = v;
+    if (v == 64 || v == 128) m->gemm_variant = v == 64 ? t5k::GEMM_256X64 : t5k::GEMM_256X128;
   }
   if (const char* e = getenv("T5H_GEMM_TAIL")) {
     const int v = atoi(e);
-    if (v >= 0 && v <= 4) m->gemm_tail_override = v;
+    if (v >= 0 && v <= 4)
+      m->gemm_variant = v == 0 ? t5k::GEMM_256X128 : v % 2 ? t5k::GEMM_64X128 : t5k::GEMM_128X128;
+  }
+  if (const char* e = getenv("T5H_GEMM_MB")) {
+    const int v = atoi(e);
+    if (v == 3 || v == 4) m->gemm_variant = v == 3 ? t5k::GEMM_192X128 : t5k::GEMM_256X128;
   }
   if (const char* e = getenv("T5H_FOLD_NORM")) m->fold_norm_off = atoi(e) == 0;
   if (const char* e = getenv("T5H_GATED_MW8")) m->gated_mw8 = atoi(e) != 0;
@@ -1658,6 +1682,18 @@ int create_impl(const void* gguf, size_t len, const t5h_config* cfg, int hip_dev
   }
   bind(m->proj);
   HIP_OK(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking));
+  {
+    std::vector<Linear*> ls;
+    for (auto& Ly : m->layers) {
+      if (Ly.fused_qkv) ls.push_back(&Ly.qkv);
+      else ls.insert(ls.end(), {&Ly.q, &Ly.k, &Ly.v});
+      ls.insert(ls.end(), {&Ly.o, &Ly.wi0, &Ly.wo});
+      if (cfg->feed_forward_gated) ls.push_back(&Ly.wi1);
+    }
+    ls.push_back(&m->proj);
+    if ((rc = build_tiled(m.get(), ls, &m->tw))) return rc;
+    HIP_OK(hipStreamSynchronize(m->stream));
+  }
   if (hipHostMalloc((void**)&m->err_host, 256, hipHostMallocMapped) != hipSuccess)
     return fail(T5H_ERR_NOMEM, "pinned flag allocation failed");
   memset(m->err_host, 0, 256);
@@ -1923,6 +1959,8 @@ int build_bf16_layers(t5h_model* m) {
     }
     L->fmt = WF_F16;
   }
+  int rc;
+  if ((rc = build_tiled(m, dense, &m->twb))) return rc;
   HIP_OK(hipStreamSynchronize(m->stream));
   m->layers_bf = std::move(lb);
   return T5H_OK;
@@ -2056,7 +2094,7 @@ int t5h_replay_kernel(t5h_model* m, int32_t kind, int32_t reps, double* avg_us) 
     return fail(T5H_ERR_INVALID, std::string("replay: no profiled forward launched ") + kKernelNames[kind]);
   auto launch = [&]() -> hipError_t {
     switch (r.type) {
-      case ReplayRec::GEMM: return t5k::launch_gemm(r.epi, r.wfmt, r.plan, r.ga, m->stream);
+      case ReplayRec::GEMM: return t5k::launch_gemm(r.epi, r.plan, r.ga, m->stream);
       case ReplayRec::GEMV: return t5k::launch_gemv(r.epi, r.wfmt, r.ga, m->stream);
       case ReplayRec::ATTN: return t5k::launch_attention(r.aa, r.n, r.D, m->stream);
       case ReplayRec::FFN: return t5k::launch_ffn_fused(r.fa, r.wfmt, m->stream);
@@ -2072,7 +2110,7 @@ int t5h_replay_kernel(t5h_model* m, int32_t kind, int32_t reps, double* avg_us) 
             t5k::launch_q8k_quantize(r.x, r.gamma, r.eps, r.n, r.D, nullptr, m->stream,
                                      reinterpret_cast<int8_t*>(r.xn), r.hd8, r.hbs);
         if (e != hipSuccess) return e;
-        return t5k::launch_gemm_hybrid(r.epi, r.plan, r.ga, m->stream);
+        return t5k::launch_gemm_hybrid(r.epi, r.hplan, r.ga, m->stream);
       }
       default: return hipErrorInvalidValue;
     }
