@@ -119,6 +119,32 @@ def test_matmul_t_q4_within_f32_summation_bound(codec, M, N, D):
     assert np.all(np.abs(got - want) <= bound)
 
 
+# the streaming kernel's passes and edges: one column short of and past a 32-column tile, a lane's
+# four columns cut at 1..3, one row in the last pass, the smallest and a long stream, both store kinds
+Q4_STREAM_SHAPES = [(33, 512), (1, 513), (16, 514), (64, 515), (32, 4095), (65, 4097), (50, 9001), (17, 65537),
+                    (33, 65536), (100, 30752)]
+
+
+@pytest.mark.parametrize("M,N", Q4_STREAM_SHAPES)
+def test_matmul_t_q4_stream_edges(codec, M, N):
+    """Device scores into a buffer with a guard on both sides, at 16-byte and at 4-byte alignment:
+    within the f32 summation bound and not a value outside the M x N block."""
+    import torch
+    rng = np.random.default_rng(M * 131 + N)
+    a = _unit_rows(M, 128, rng)
+    codes = rng.integers(0, 256, (N, 64)).astype(np.uint8)
+    r = orc.residual_decode(codes, 128).astype(np.float64)
+    want = a.astype(np.float64) @ r.T
+    bound = 128 * 2.0 ** -23 * (np.abs(a).astype(np.float64) @ np.abs(r).T) + 1e-30
+    da, dc = torch.from_numpy(a).cuda(), torch.from_numpy(codes).cuda()
+    for off in (64, 65):
+        c = torch.full((off + M * N + 64,), 7.5, device="cuda")
+        codec.matmul_t_q4_device(da.data_ptr(), M, dc.data_ptr(), N, 128, c.data_ptr() + 4 * off)
+        c = c.cpu().numpy()
+        assert np.all(np.abs(c[off:off + M * N].reshape(M, N) - want) <= bound)
+        assert np.all(c[:off] == 7.5) and np.all(c[off + M * N:] == 7.5)
+
+
 def test_matmul_t_q4_matches_decode_then_matmul(codec):
     """Same scores as the reference's two steps, from_companded_q4_bytes then matmul_t."""
     from witchcraft_amd import score

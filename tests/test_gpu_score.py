@@ -70,6 +70,30 @@ def test_matmul_t_vs_oracle(score, M, N, D, bf16_b):
     assert np.all(np.isfinite(got))
 
 
+# the streaming kernel's passes and edges: one column short of and past a 32-column tile, a lane's
+# four columns cut at 1..3, one row in the last pass, the last row count of its range, both store kinds
+STREAM_SHAPES = [(33, 512), (1, 513), (16, 514), (64, 515), (32, 4095), (65, 4097), (17, 65537), (33, 65536),
+                 (128, 16416)]
+
+
+@pytest.mark.parametrize("bf16_b", [False, True])
+@pytest.mark.parametrize("M,N", STREAM_SHAPES)
+def test_matmul_t_stream_edges(score, M, N, bf16_b):
+    """Device scores into a buffer with a guard on both sides, at 16-byte and at 4-byte alignment:
+    within the f32 summation bound and not a value outside the M x N block."""
+    import torch
+    a, b = _data(M, N, 128, seed=M * 31 + N)
+    want = orc.matmul_t(a, b, bf16_b=bf16_b).astype(np.float64)
+    bound = _bound(a, b, bf16_b)
+    da, db = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    for off in (64, 65):
+        c = torch.full((off + M * N + 64,), 7.5, device="cuda")
+        score.matmul_t_device(da.data_ptr(), M, db.data_ptr(), N, 128, c.data_ptr() + 4 * off, bf16_b=bf16_b)
+        c = c.cpu().numpy()
+        assert np.all(np.abs(c[off:off + M * N].reshape(M, N) - want) <= bound)
+        assert np.all(c[:off] == 7.5) and np.all(c[off + M * N:] == 7.5)
+
+
 def test_matmul_t_d_zero_is_zero(score):
     a = np.zeros((5, 0), np.float32)
     b = np.zeros((9, 0), np.float32)

@@ -37,6 +37,7 @@ using t5k::Q4Table;
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kBufDword3 = 0x00020000;  // raw buffer descriptor word 3: 32-bit data, OOB -> 0
+constexpr int kBufNt = 2;               // buffer access policy bit: non-temporal
 
 // The code of r: the number of thresholds t[0..14] (strictly increasing) at or below r, found
 // by bisection -- 4 compares instead of 15.  code >= 8 iff r >= t[7]; then, from base i,
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(256) void residual_decode_kernel(const uint8_t* __r
   for (int j = 0; j < 2 * n; j++) out[2 * i + j] = v[j];
 }
 
-// Query-sized A (M <= 32 rows, D = 128) against N coded residual rows: the stream of
+// Query-sized A (16 MB <= 32 rows per grid row, D = 128) against N coded residual rows: the stream of
 // matmul_t_stream_kernel (k_score.hip) over 64-byte code rows.  Wave w takes 32-row tiles
 // w, w + W, ...; lane (lr, lg) owns rows lr and 16 + lr of a tile and their values
 // k = 32 lg .. 32 lg + 31 (16 contiguous code bytes), which it feeds to the MFMAs as
@@ -170,8 +171,17 @@ __device__ __forceinline__ void q4_stream_f32(const float* __restrict__ A, const
       const bool row_ok = 16 * i + lr < M;
 #pragma unroll
       for (int nb = 0; nb < 2; nb++)
-        if (row_ok && 32 * t + 16 * nb + 4 * lg < N)
+        if (row_ok && 32 * t + 16 * nb + 4 * lg + 3 < N)
           __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, 0);
+      if (t >= nfull && row_ok)
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) {  // the last tile: N may end inside a lane's four columns
+          const int left = N - (32 * t + 16 * nb + 4 * lg);
+#pragma unroll
+          for (int j = 0; j < 3; j++)
+            if (left < 4 && j < left)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][nb][j]), rs, soff[i] + 64 * nb + 4 * j, 0, 0);
+        }
     }
   };
   // Same issue order as matmul_t_stream_kernel: next tile's loads, previous tile's stores,
@@ -209,7 +219,9 @@ __global__ __launch_bounds__(256, 2) void matmul_t_q4_stream_kernel(const float*
                                                                     const uint8_t* __restrict__ codes, Q4Table tab,
                                                                     float* __restrict__ C, int M, int N) {
   __shared__ Q4StreamLds<MB> sh;
-  q4_stream_f32<MB>(A, codes, tab, C, M, N, sh);
+  A += (size_t)blockIdx.y * 16 * MB * 128;
+  C += (size_t)blockIdx.y * 16 * MB * N;
+  q4_stream_f32<MB>(A, codes, tab, C, min(M - (int)blockIdx.y * 16 * MB, 16 * MB), N, sh);
 }
 
 // The same stream on bf16 MFMAs.  v_mfma_f32_16x16x32_bf16 runs 8x the FLOPs of
@@ -244,11 +256,15 @@ __device__ __forceinline__ void split3(float x, uint32_t& hi, uint32_t& mid, uin
   lo = bf16_rne_bits(r2);
 }
 
-template <int MB>
+template <int MB, bool NT>
 __global__ __launch_bounds__(256, 2) void matmul_t_q4_split_kernel(const float* __restrict__ A,
                                                                    const uint8_t* __restrict__ codes, Q4Table tab,
                                                                    float* __restrict__ C, int M, int N) {
   constexpr int D = 128;
+  // 16 MB query rows per grid row
+  A += (size_t)blockIdx.y * 16 * MB * D;
+  C += (size_t)blockIdx.y * 16 * MB * N;
+  M = min(M - (int)blockIdx.y * 16 * MB, 16 * MB);
   __shared__ uint4 pt[256];
   __shared__ Q4StreamLds<MB> sh;
   __shared__ int bad;
@@ -350,8 +366,17 @@ __global__ __launch_bounds__(256, 2) void matmul_t_q4_split_kernel(const float* 
       const bool row_ok = 16 * i + lr < M;
 #pragma unroll
       for (int nb = 0; nb < 2; nb++)
-        if (row_ok && 32 * t + 16 * nb + 4 * lg < N)
-          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, 0);
+        if (row_ok && 32 * t + 16 * nb + 4 * lg + 3 < N)
+          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, NT ? kBufNt : 0);
+      if (t >= nfull && row_ok)
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) {  // the last tile: N may end inside a lane's four columns
+          const int left = N - (32 * t + 16 * nb + 4 * lg);
+#pragma unroll
+          for (int j = 0; j < 3; j++)
+            if (left < 4 && j < left)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][nb][j]), rs, soff[i] + 64 * nb + 4 * j, 0, 0);
+        }
     }
   };
   // the f32 kernel's issue order: next tile's loads, previous tile's stores, this tile's MFMAs
@@ -477,21 +502,38 @@ hipError_t launch_residual_decode(const uint8_t* codes, size_t nbytes, const Q4T
 hipError_t launch_matmul_t_q4(const float* A, const uint8_t* codes, const Q4Table& tab, float* C, int M, int N,
                               int D, hipStream_t s) {
   if (M <= 0 || N <= 0) return hipSuccess;
-  const bool aligned = ((uintptr_t)A & 15) == 0 && ((uintptr_t)codes & 15) == 0 && ((uintptr_t)C & 15) == 0;
-  if (D == 128 && M <= 32 && N % 4 == 0 && N >= 4096 && aligned && (size_t)N * 4 * 32 < 0x7fffffffu) {
+  // A long stream of 128-d codes takes the streaming kernels in passes of 32 query rows, at any N:
+  // split kernel / tiled kernel below: 32 x 1,000 8.8 / 9.9 us, 32 x 131,071 18.8 / 30, 50 x 200,000
+  // 34 / 77, 32 x 1,048,575 78 / 226, 1,000 x 16,384 73 / 98.  (Scores may start on any f32: 16-byte
+  // buffer stores need 4-byte alignment only.)
+  const bool aligned = ((uintptr_t)A & 15) == 0 && ((uintptr_t)codes & 15) == 0;
+  const int mb = M <= 16 ? 1 : 2, passes = M <= 16 ? 1 : (M + 31) / 32;
+  if (D == 128 && N >= 512 && passes <= 65535 && aligned && (size_t)N * 4 * 32 < 0x7fffffffu) {
     const int wgs = std::min(2 * num_cus_codec(), (N + 127) / 128);
+    // Scores as non-temporal stores where every store fills whole 128-byte lines and the scores outgrow
+    // what the L2s would keep for a reader anyway: twice the bytes of the codes at 32 rows, they otherwise
+    // evict the codes of the next tiles (32 x 1,048,576 76 -> 63 us, 16 x 262,144 17.9 -> 16.3, 32 x
+    // 65,536 12.4 -> 11.7).  Rows that start inside a line lose, each half line going out by itself (32 x
+    // 1,048,575 78 -> 131 us).
+    const bool nt = N % 32 == 0 && ((uintptr_t)C & 127) == 0 && (size_t)M * N * 4 >= (size_t)8 << 20;
     // T5H_Q4_SCORE_F32=1 keeps the f32-MFMA stream (measurement and tests)
     static const bool f32_only = [] {
       const char* e = getenv("T5H_Q4_SCORE_F32");
       return e && atoi(e) == 1;
     }();
+    const dim3 grid(wgs, passes);
+#define T5K_Q4(...) hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(256), 0, s, A, codes, tab, C, M, N)
     if (f32_only) {
-      if (M <= 16) hipLaunchKernelGGL((matmul_t_q4_stream_kernel<1>), dim3(wgs), dim3(256), 0, s, A, codes, tab, C, M, N);
-      else hipLaunchKernelGGL((matmul_t_q4_stream_kernel<2>), dim3(wgs), dim3(256), 0, s, A, codes, tab, C, M, N);
+      if (mb == 1) T5K_Q4(matmul_t_q4_stream_kernel<1>);
+      else T5K_Q4(matmul_t_q4_stream_kernel<2>);
+    } else if (mb == 1) {
+      if (nt) T5K_Q4(matmul_t_q4_split_kernel<1, true>);
+      else T5K_Q4(matmul_t_q4_split_kernel<1, false>);
     } else {
-      if (M <= 16) hipLaunchKernelGGL((matmul_t_q4_split_kernel<1>), dim3(wgs), dim3(256), 0, s, A, codes, tab, C, M, N);
-      else hipLaunchKernelGGL((matmul_t_q4_split_kernel<2>), dim3(wgs), dim3(256), 0, s, A, codes, tab, C, M, N);
+      if (nt) T5K_Q4(matmul_t_q4_split_kernel<2, true>);
+      else T5K_Q4(matmul_t_q4_split_kernel<2, false>);
     }
+#undef T5K_Q4
     return hipGetLastError();
   }
   const dim3 grid((N + 63) / 64, (M + 63) / 64);

@@ -30,6 +30,7 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 // Word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs: 32-bit data format, so
 // an access beyond num_records returns zero (loads) or is dropped (stores).
 constexpr int kBufDword3 = 0x00020000;
+constexpr int kBufNt = 2;  // buffer access policy bit: non-temporal
 
 __device__ __forceinline__ float4 ldg4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 
@@ -154,18 +155,21 @@ __global__ __launch_bounds__(256) void matmul_t_kernel(const float* __restrict__
   }
 }
 
-// Query-sized A (M <= 16 MB <= 32) against a long B of 128-d rows, N % 4 == 0
+// Query-sized A (16 MB <= 32 rows per grid row) against a long B of 128-d rows
 // (src/lib.rs:734-735): a stream over B.  Persistent waves; wave w takes 32-column tiles
 // w, w + W, w + 2W, ... (W = all waves of the grid, so the waves in flight cover one
 // contiguous stretch of B).  A sits in LDS for the whole run, and the next tile's B loads
 // are issued before the current tile's MFMAs and stores, so HBM streams while the f32
 // MFMAs run.
-template <int MB, bool BF16B>
+template <int MB, bool BF16B, bool NT>
 __global__ __launch_bounds__(256, 2) void matmul_t_stream_kernel(const float* __restrict__ A,
                                                                  const float* __restrict__ B,
                                                                  float* __restrict__ C, int M, int N) {
   constexpr int D = 128, KB = D / 16, AS = D / 4 + 1;  // A row stride in LDS: 33 float4
   __shared__ float4 As[16 * MB * AS];
+  A += (size_t)blockIdx.y * 16 * MB * D;  // this grid row's pass of query rows
+  C += (size_t)blockIdx.y * 16 * MB * N;
+  M = min(M - (int)blockIdx.y * 16 * MB, 16 * MB);
   const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
   // wave index made visibly uniform, so tile bases and descriptors live in scalar registers
   const int w0 = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = gridDim.x * 4;
@@ -214,10 +218,8 @@ __global__ __launch_bounds__(256, 2) void matmul_t_stream_kernel(const float* __
         }
       }
   };
-  // lane holds C[16 i + lr][32 t + 16 nb + 4 lg + 0..3]; N % 4 == 0, so a lane's 4 columns
-  // are all inside or all outside [0, N)
-  // (stores through a descriptor based at column 32 t; row offsets r N 4 < 2^31 is a launch
-  // condition)
+  // lane holds C[16 i + lr][32 t + 16 nb + 4 lg + 0..3] (stores through a descriptor based at
+  // column 32 t; row offsets r N 4 < 2^31 is a launch condition)
   int soff[MB];
 #pragma unroll
   for (int i = 0; i < MB; i++) soff[i] = ((16 * i + lr) * N + 4 * lg) * 4;
@@ -229,8 +231,17 @@ __global__ __launch_bounds__(256, 2) void matmul_t_stream_kernel(const float* __
       const bool row_ok = 16 * i + lr < M;
 #pragma unroll
       for (int nb = 0; nb < 2; nb++)
-        if (row_ok && 32 * t + 16 * nb + 4 * lg < N)
-          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, 0);
+        if (row_ok && 32 * t + 16 * nb + 4 * lg + 3 < N)
+          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, NT ? kBufNt : 0);
+      if (t >= nfull && row_ok)
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) {  // the last tile: N may end inside a lane's four columns
+          const int left = N - (32 * t + 16 * nb + 4 * lg);
+#pragma unroll
+          for (int j = 0; j < 3; j++)
+            if (left < 4 && j < left)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][nb][j]), rs, soff[i] + 64 * nb + 4 * j, 0, 0);
+        }
     }
   };
   // Per tile: issue the next tile's loads, then the previous tile's stores, then this tile's
@@ -726,16 +737,30 @@ hipError_t launch_matmul_t(const float* A, const float* B, float* C, int M, int 
   if (tiles_n * tiles_m > 0x7fffffffL) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tiles_n * tiles_m));
   const bool vec = D % 4 == 0 && aligned16(A) && aligned16(B) && aligned16(C);
-  if (vec && D == 128 && M <= 32 && N >= 4096 && N % 4 == 0 && 32L * N * 4 < (1L << 31)) {
-    // query x residuals: persistent streaming kernel, 2 workgroups per CU
-    const int wgs = (int)std::min<long>(2L * num_cus(), (N + 127) / 128);
+  // Few rows of A against a long B: the persistent streaming kernel, 2 workgroups per CU, in passes of
+  // 32 rows.  Streaming kernel / tiled kernel: 32 x 1,000 8.3 / 9.5 us, 50 x 16,384 8.5 / 15.7,
+  // 50 x 200,000 50 / 64, 64 x 200,001 60 / 84, 128 x 4,096 9.3 / 15.7; from 256 rows on B is read again
+  // once too often (256 x 16,384 19.5 / 19.1, 1,000 x 50,000 215 / 182).
+  const bool rows16 = D % 4 == 0 && aligned16(A) && aligned16(B);
+  if (rows16 && D == 128 && M <= 128 && N >= 512 && 32L * N * 4 < (1L << 31)) {
+    const int passes = mb == 1 ? 1 : (M + 31) / 32;
+    const dim3 g((unsigned)std::min<long>(2L * num_cus(), (N + 127) / 128), (unsigned)passes);
+    // scores past the caches as they are written: a store of whole 128-byte lines, and more of them than
+    // the L2s would hold for a reader (16 x 262,144 34.9 -> 33.4 us, 32 x 1,048,576 140.5 -> 137; a row
+    // that starts inside a line loses: see matmul_t_q4's rule)
+    const bool nt = N % 32 == 0 && ((uintptr_t)C & 127) == 0 && (size_t)M * N * 4 >= (size_t)8 << 20;
+#define T5K_STREAM(MBV, BF, NT) \
+  hipLaunchKernelGGL((matmul_t_stream_kernel<MBV, BF, NT>), g, dim3(256), 0, s, A, B, C, M, N)
+#define T5K_STREAM_NT(MBV, BF) \
+  if (nt) T5K_STREAM(MBV, BF, true); \
+  else T5K_STREAM(MBV, BF, false)
     if (mb == 1) {
-      if (bf16_b) hipLaunchKernelGGL((matmul_t_stream_kernel<1, true>), dim3(wgs), dim3(256), 0, s, A, B, C, M, N);
-      else hipLaunchKernelGGL((matmul_t_stream_kernel<1, false>), dim3(wgs), dim3(256), 0, s, A, B, C, M, N);
+      if (bf16_b) { T5K_STREAM_NT(1, true); } else { T5K_STREAM_NT(1, false); }
     } else {
-      if (bf16_b) hipLaunchKernelGGL((matmul_t_stream_kernel<2, true>), dim3(wgs), dim3(256), 0, s, A, B, C, M, N);
-      else hipLaunchKernelGGL((matmul_t_stream_kernel<2, false>), dim3(wgs), dim3(256), 0, s, A, B, C, M, N);
+      if (bf16_b) { T5K_STREAM_NT(2, true); } else { T5K_STREAM_NT(2, false); }
     }
+#undef T5K_STREAM_NT
+#undef T5K_STREAM
     return hipGetLastError();
   }
 #define T5K_MMT(MBV, BF, VEC) \
