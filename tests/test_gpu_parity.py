@@ -181,6 +181,20 @@ def test_small_model_ragged_batch_past_four_key_tiles(small):
     _check_batch(gpu, ora, ids, cu)
 
 
+@pytest.mark.parametrize("tiles", [3, 5, 6, 7, 8])
+def test_small_model_last_key_tile_of_a_long_sequence(small, tiles):
+    """Only a sequence's last key tile is loaded with its rows clamped, the others through shared
+    offsets: 1, 31, 32, 33, 63 and 64 keys in the last of `tiles` tiles, followed in memory by rows
+    of another sequence, in both orders of the batch."""
+    cfg, _, gpu, ora = small
+    rng = np.random.default_rng(tiles)
+    lens = np.array([64 * (tiles - 1) + k for k in (1, 31, 32, 33, 63, 64)])
+    for order in (lens, lens[::-1]):
+        cu = np.concatenate([[0], np.cumsum(order)]).astype(np.int32)
+        ids = rng.integers(1, cfg["vocab_size"], size=int(cu[-1])).astype(np.uint32)
+        _check_batch(gpu, ora, ids, cu)
+
+
 def test_small_model_max_length_sequence(small):
     cfg, _, gpu, ora = small
     ids = np.random.default_rng(2).integers(1, cfg["vocab_size"], size=2048).astype(np.uint32)

@@ -16,6 +16,13 @@
 // are issued two tiles ahead; one barrier per tile.  A sequence of at most 128 tokens takes a
 // path with 64-query work items and 16-query waves instead (small_sequence).
 //
+// What bounds it: issue of vector instructions beside the matrix core.  A full tile costs a wave 130
+// vector instructions (32 exp at half rate) and 16 MFMAs of 32 clocks; per SIMD the three waves took
+// 1,329 clocks a tile with 172 vector instructions (850 + 512 clocks of the two units, hardly
+// overlapped) and take about 1,250 with 130: 18 windows of 2,048 tokens, 12 heads, in two launches,
+// 129 + 140 us -> 122 + 131.  Two waves per SIMD with the next tile's scores beside this tile's
+// softmax were slower (138 + 150), s_setprio around the MFMAs changed nothing.
+//
 // The score block is computed transposed, S^T = K . Q^T (32 keys x 32 queries per MFMA), so
 // that the accumulator layout (lane = query column; lane half h holds keys 8a + 4h + b) is, four
 // registers at a time, the B operand of O^T = V^T . P^T with the keys of each 16-key step taken
@@ -94,31 +101,56 @@ __device__ __forceinline__ void lds_load4(const void* base, uint32_t voff, uint3
 // `nrows` repeat the last row of the sequence: finite values, which the masked scores (P = 0)
 // then ignore.
 template <int R>
+__device__ __forceinline__ uint32_t dma_offset(int j, int nrows, int wave, int lane) {
+  const int row = 16 * wave + 8 * j + (lane >> 3);
+  const int chunk = (lane ^ rot<R>(row)) & 7;
+  const int srow = row < nrows ? row : nrows - 1;
+  return (uint32_t)(srow * (DK * 2) + chunk * 16);
+}
+template <int R>
 __device__ __forceinline__ void dma_tile(const _Float16* src, int nrows, _Float16* dst, int wave, int lane) {
 #pragma unroll
+  for (int j = 0; j < 2; j++)
+    lds_load16(src, dma_offset<R>(j, nrows, wave, lane), lds_offset(dst + (16 * wave + 8 * j) * DK));
+}
+// The same for a tile whose 64 rows all lie in the sequence: ofs = dma_offset<R>(0, KT, ..) is the
+// same for every such tile, so a caller with many of them forms it once.  Eight rows further on
+// ROT_K has bit 1 flipped (chunk ^ 2: 32 bytes), ROT_V and ROT_8 repeat.
+template <int R>
+__device__ __forceinline__ void dma_full_tile(const _Float16* src, uint32_t ofs, _Float16* dst, int wave) {
+  lds_load16(src, ofs, lds_offset(dst + 16 * wave * DK));
+  lds_load16(src + 8 * DK, R == ROT_K ? ofs ^ 32 : ofs, lds_offset(dst + (16 * wave + 8) * DK));
+}
+// The last tile of a sequence from the same offsets: row = ofs / 128, clamped as in dma_offset.
+// (The empty asm keeps the parts of ofs from being held in registers through the key loop.)
+template <int R>
+__device__ __forceinline__ void dma_last_tile(const _Float16* src, uint32_t ofs, int nrows, _Float16* dst, int wave) {
+  asm volatile("" : "+v"(ofs));
+#pragma unroll
   for (int j = 0; j < 2; j++) {
-    const int row = 16 * wave + 8 * j + (lane >> 3);
-    const int chunk = (lane ^ rot<R>(row)) & 7;
-    const int srow = row < nrows ? row : nrows - 1;
-    lds_load16(src, (uint32_t)(srow * (DK * 2) + chunk * 16), lds_offset(dst + (16 * wave + 8 * j) * DK));
+    const int srow = min((int)(ofs >> 7) + 8 * j, nrows - 1);
+    const uint32_t chunk = (R == ROT_K && j ? ofs ^ 32 : ofs) & 127;
+    lds_load16(src, (uint32_t)srow * 128 | chunk, lds_offset(dst + (16 * wave + 8 * j) * DK));
   }
 }
 
-// Per-lane LDS offsets (f16 elements from a tile's base) of the operand reads.
+// Per-lane LDS offsets (bytes from a tile's base) of the operand reads.
 // k[ds]: the K operand of dims 16 ds .. +15 for key half 0 (key row l % 32, dims + 8 (l / 32));
 // half kb adds 32 rows.  v[db]: the V^T operand of dims 32 db .. +31 for key step 0 (below);
 // step c adds 16 rows, its second 8 keys another 8.  Rows that differ by a multiple of 8 share
 // their rotation, so those additions are constants that fold into the reads' immediate offsets.
+// b: the staged bias of (key 4 h of the tile, the lane's query), (j - qi) - (k0 - q0 - (QT - 1)).
 struct LaneOfs {
-  int k[4], v[2];
+  int k[4], v[2], b;
 };
-__device__ __forceinline__ LaneOfs lane_offsets(int lane) {
+__device__ __forceinline__ LaneOfs lane_offsets(int lane, int wave) {
   const int l32 = lane & 31, h = lane >> 5, i = lane & 15, g = lane >> 4;
   LaneOfs o;
 #pragma unroll
-  for (int ds = 0; ds < 4; ds++) o.k[ds] = swz<ROT_K>(l32, 16 * ds + 8 * h);
+  for (int ds = 0; ds < 4; ds++) o.k[ds] = 2 * swz<ROT_K>(l32, 16 * ds + 8 * h);
 #pragma unroll
-  for (int db = 0; db < 2; db++) o.v[db] = swz<ROT_V>(4 * h + (i >> 2), 32 * db + 16 * (g & 1) + 4 * (i & 3));
+  for (int db = 0; db < 2; db++) o.v[db] = 2 * swz<ROT_V>(4 * h + (i >> 2), 32 * db + 16 * (g & 1) + 4 * (i & 3));
+  o.b = 4 * ((QT - 1) - wave * QW - l32 + 4 * h);
   return o;
 }
 
@@ -129,8 +161,9 @@ __device__ __forceinline__ LaneOfs lane_offsets(int lane) {
 // read returns column c0 + n of those 4 rows to lane n.
 __device__ __forceinline__ h8 v_operand(const _Float16* Vb, int c, int vo) {
   typedef __attribute__((address_space(3))) s4v lds_s4;
-  const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(Vb + vo + 16 * c * DK));
-  const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(Vb + vo + (16 * c + 8) * DK));
+  const char* v = reinterpret_cast<const char*>(Vb) + vo;
+  const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(v + 2 * 16 * c * DK));
+  const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(v + 2 * (16 * c + 8) * DK));
   h8 r;
   __builtin_memcpy(&r, &lo, 8);
   __builtin_memcpy(reinterpret_cast<char*>(&r) + 8, &hi, 8);
@@ -146,22 +179,23 @@ __device__ __forceinline__ h8 v_operand(const _Float16* Vb, int c, int vo) {
 // The reference max moves only when needed.  A query's scores lie in two lanes (the two key
 // halves of each 8-key group), so its tile max is one permlane32 swap away; the reference
 // m_run is moved to the running max, and O and l rescaled, only when some query's tile max
-// exceeds m_run by more than 14 / log2(e) (always on the first tile, where m_run = -inf), so
+// exceeds m_run by more than 14 / log2(e), i.e. m_lim (always on the first tile, where both are -inf), so
 // every P = 2^((s - m_run) log2e) stays at most 2^14, well inside f16.  Same result up to
 // rounding: P and l carry the same factor, divided out at the end, and m_run is a score
 // already seen, so l >= 1.  A rescale on every tile measured slower.  l sums the f16 P that the
 // P.V product uses; it is kept per lane (this lane's keys) and reduced across the two lanes of
 // a query only at the end.
 template <bool FULL, bool MASK>
-__device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* Vb, const float* Bsb, int bofs,
-                                          LaneOfs lo, const h8 (&qf)[4], bool qv, int k0, int L, float& m_run,
+__device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* Vb, const float* Bsb, LaneOfs& lo,
+                                          const h8 (&qf)[4], bool qv, int k0, int L, float& m_run, float& m_lim,
                                           float& l_run, f16v (&o)[2]) {
   constexpr int NS = FULL ? 2 : 1;  // 32-key halves with keys < L
   const int h = (threadIdx.x >> 5) & 1;
-  // The offsets pass through an empty asm, so the compiler keeps these eight lane values and
+  // The offsets pass through an empty asm, so the compiler keeps these seven lane values and
   // folds each ring slot's base into the reads' immediate offsets, rather than holding a
-  // precomputed address per slot.
-  asm volatile("" : "+v"(bofs), "+v"(lo.k[0]), "+v"(lo.k[1]), "+v"(lo.k[2]), "+v"(lo.k[3]), "+v"(lo.v[0]),
+  // precomputed address per slot.  (The caller's own values are redefined: a copy of them would
+  // cost seven moves a tile.)
+  asm volatile("" : "+v"(lo.b), "+v"(lo.k[0]), "+v"(lo.k[1]), "+v"(lo.k[2]), "+v"(lo.k[3]), "+v"(lo.v[0]),
                "+v"(lo.v[1]));
   // S^T[key][query] + bias: register r of half kb holds key 32 kb + 8 (r / 4) + 4 h + r % 4.
   // The accumulators start from the bias, so the matrix core does the add.  The lane's bias
@@ -169,7 +203,7 @@ __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* V
   // pair up as ds_read2_b32 with immediate offsets from that one register; a slot base too large
   // for those offsets would otherwise be added per pair.
   typedef const __attribute__((address_space(3))) float lds_f;
-  uint32_t baddr = lds_offset(Bsb) + 4u * (uint32_t)bofs;
+  uint32_t baddr = lds_offset(Bsb) + (uint32_t)lo.b;
   asm volatile("" : "+v"(baddr));
   lds_f* bsrc = (lds_f*)(uintptr_t)baddr;
   f16v s[NS];
@@ -184,7 +218,7 @@ __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* V
 #pragma unroll
   for (int ds = 0; ds < 4; ds++)
 #pragma unroll
-    for (int kb = 0; kb < NS; kb++) ka[ds][kb] = *reinterpret_cast<const h8*>(&Ksb[lo.k[ds] + 32 * kb * DK]);
+    for (int kb = 0; kb < NS; kb++) ka[ds][kb] = *reinterpret_cast<const h8*>(reinterpret_cast<const char*>(Ksb) + lo.k[ds] + 2 * 32 * kb * DK);
 #pragma unroll
   for (int ds = 0; ds < 4; ds++)
 #pragma unroll
@@ -207,16 +241,18 @@ __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* V
   for (int kb = 0; kb < NS; kb++)
 #pragma unroll
     for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[kb][r]);
-  mx = max_xor32(mx);  // finite: key k0 < L is valid
-  // Only lanes of queries below L take part (qv), so that whatever the rows past L hold cannot
-  // change when the valid queries rescale: the result stays independent of the batch around
-  // the sequence.  !(x <= 14) also catches NaN.
-  if (__any(qv && !((mx - m_run) * LOG2E <= 14.f))) {
+  // mx is the max of this lane's half of the keys; some lane of a query exceeds m_lim exactly if
+  // the query's max does, so the lanes only meet in the branch.  m_lim is +inf for queries past
+  // L, so that whatever those rows hold cannot change when the valid queries rescale: the result
+  // stays independent of the batch around the sequence.
+  if (__builtin_amdgcn_ballot_w64(mx > m_lim)) {
+    mx = max_xor32(mx);  // finite: key k0 < L is valid
     // the rescale of O sits in a branch of its own, so the accumulators keep their registers
     const float m_new = fmaxf(m_run, mx);
     // 1 where the max did not move, 0 on the first tile (O and l are still 0 there)
     const float corr = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E);
     m_run = m_new;
+    m_lim = qv ? m_new + 14.f / LOG2E : INFINITY;
     l_run *= corr;
 #pragma unroll
     for (int db = 0; db < 2; db++) o[db] *= corr;
@@ -233,6 +269,8 @@ __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* V
 #pragma unroll
     for (int j = 0; j < 8; j++)
       pb[j] = (_Float16)__builtin_amdgcn_exp2f(__builtin_fmaf(s[c >> 1][8 * (c & 1) + j], LOG2E, mb));
+    // packed once: without the empty asm the compiler converts and packs again for the sums
+    asm("" : "+v"(pb));
 #pragma unroll
     for (int j = 0; j < 8; j += 2) l_run = __builtin_amdgcn_fdot2(h2{pb[j], pb[j + 1]}, ones, l_run, false);
 #pragma unroll
@@ -393,14 +431,20 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
   // A tile's loads, the same five per wave for every tile: K and V rows k0.. (clamped to the
   // sequence) and 64 of the bias values of distances k0 - q0 - (QT - 1) .. (QT + KT - 1 of the
   // 256 staged are read).
+  const uint32_t kofs = dma_offset<ROT_K>(0, KT, wave, lane), vofs = dma_offset<ROT_V>(0, KT, wave, lane);
   auto load_tile = [&](int k0, _Float16* Kd, _Float16* Vd, float* Bd) __attribute__((always_inline)) {
-    dma_tile<ROT_K>(Kg + (size_t)k0 * DK, L - k0, Kd, wave, lane);
-    dma_tile<ROT_V>(Vg + (size_t)k0 * DK, L - k0, Vd, wave, lane);
+    if (k0 + KT <= L) {
+      dma_full_tile<ROT_K>(Kg + (size_t)k0 * DK, kofs, Kd, wave);
+      dma_full_tile<ROT_V>(Vg + (size_t)k0 * DK, vofs, Vd, wave);
+    } else {
+      dma_last_tile<ROT_K>(Kg + (size_t)k0 * DK, kofs, L - k0, Kd, wave);
+      dma_last_tile<ROT_V>(Vg + (size_t)k0 * DK, vofs, L - k0, Vd, wave);
+    }
     lds_load4(lut + (k0 - q0 - (QT - 1) + 64 * wave), 4u * lane, lds_offset(Bd + 64 * wave));
   };
   static_assert(LOADS == 5, "the wait below counts five loads per tile");
 
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, m_lim = qi < L ? -INFINITY : INFINITY, l_run = 0.f;
   f16v o[2];
 #pragma unroll
   for (int db = 0; db < 2; db++)
@@ -408,9 +452,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
     for (int r = 0; r < 16; r++) o[db][r] = 0.f;
 
   const int ntile = (L + KT - 1) / KT;
-  // Bs index of this lane's (key 4h + r of the tile, query qi): (j - qi) - (k0 - q0 - (QT - 1))
-  const int bofs = (QT - 1) - wave * QW - l32 + 4 * h;
-  const LaneOfs lofs = lane_offsets(lane);
+  LaneOfs lofs = lane_offsets(lane, wave);
   // Tile t lives in slot t % 3.  Step t waits for this wave's loads of tile t (those of t + 1
   // may still be in flight), meets the other waves (every wave's part of tile t has landed, and
   // every wave is done with tile t - 1), issues tile t + 2 into the slot tile t - 1 used, then
@@ -426,9 +468,14 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
     if (t + 2 < ntile) load_tile((t + 2) * KT, next.k, next.v, next.b);
     if (!decltype(act)::value) return;
     const int k0 = t * KT;
-    if (!last) attn_tile<true, false>(cur.k, cur.v, cur.b, bofs, lofs, qf, qi < L, k0, L, m_run, l_run, o);
-    else if (L - k0 > 32) attn_tile<true, true>(cur.k, cur.v, cur.b, bofs, lofs, qf, qi < L, k0, L, m_run, l_run, o);
-    else attn_tile<false, true>(cur.k, cur.v, cur.b, bofs, lofs, qf, qi < L, k0, L, m_run, l_run, o);
+    if (!decltype(tail)::value) {
+      attn_tile<true, false>(cur.k, cur.v, cur.b, lofs, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
+      return;
+    }
+    LaneOfs lt = lofs;  // (three variants that redefine one set of offsets would spill)
+    if (!last) attn_tile<true, false>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
+    else if (L - k0 > 32) attn_tile<true, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
+    else attn_tile<false, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
   };
   // The Q loads complete before tile 0, which is peeled off the loop, so that the loop body (whose
   // steps are never the last tile) carries a single tile variant and no wait on them.
@@ -462,7 +509,10 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
   else run(std::false_type{});
   l_run = sum_xor32(l_run);
 
-  if (active && qi < L) {  // written in operand order for the O GEMM
+  // (the lane's query again, from the lane's number: held through the key loop it would spill)
+  const int le = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  const int qe = q0 + wave * QW + (le & 31), he = le >> 5;
+  if (active && qe < L) {  // written in operand order for the O GEMM
     const float inv = 1.0f / l_run;
     const int inner = p.heads * DK;
 #pragma unroll
@@ -471,7 +521,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
       for (int a = 0; a < 4; a++) {
         const h4 v = {(_Float16)(o[db][4 * a] * inv), (_Float16)(o[db][4 * a + 1] * inv),
                       (_Float16)(o[db][4 * a + 2] * inv), (_Float16)(o[db][4 * a + 3] * inv)};
-        *reinterpret_cast<h4*>(p.out + tiled_index(s0 + qi, hd * DK + 32 * db + 8 * a + 4 * h, inner)) = v;
+        *reinterpret_cast<h4*>(p.out + tiled_index(s0 + qe, hd * DK + 32 * db + 8 * a + 4 * he, inner)) = v;
       }
   }
 }
