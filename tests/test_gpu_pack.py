@@ -128,6 +128,21 @@ def test_coder_lengths_and_histograms(codec, rows, cols, kind):
         assert got.view(np.uint32).tolist() == want.view(np.uint32).tolist()
 
 
+@pytest.mark.parametrize("rows,cols,big", [(31, 128, 2.0), (32, 128, 8.0), (33, 128, 40.0), (65, 64, 150.0),
+                                           (96, 32, 300.0), (512, 128, 900.0), (9, 250, 2500.0)])
+def test_symbols_across_the_counters(codec, rows, cols, big):
+    """Rows around the column sums' blocks of 32, and values past 1 (scaled by the largest one below 1)
+    whose symbols fall on both sides of the per-lane counters (64), of the first histogram pass (8,192)
+    and of the 16 bits a symbol is stored in: the oracle's bytes."""
+    rng = np.random.default_rng(rows)
+    x = _emb(rows, cols, rows)
+    at = rng.integers(0, x.size, 12)
+    x.reshape(-1)[at] = np.linspace(1.0, big, at.size).astype(np.float32) * rng.choice([-1, 1], at.size)
+    buf = _or_refused(orc.embeddings_to_packed, x)
+    assert buf != "refused"
+    assert codec.embeddings_to_packed(x) == buf
+
+
 @pytest.mark.parametrize("delta", [-1, -3, 1])
 def test_histogram_totals_other_than_the_slots(codec, delta):
     """A frequency changed in the stored histogram: slots left uncovered decode as the oracle

@@ -60,8 +60,18 @@ __global__ __launch_bounds__(256) void pk_colsort(const float* __restrict__ x, P
   perm_out[(size_t)blockIdx.x * 256 + c] = c < cols ? c : 0;
   if (c < cols) {
     const float* p = x + (size_t)w.row0 * cols + c;
-    float s = 0.f;
-    for (int r = 0; r < w.rows; r++) s += p[(size_t)r * cols];
+    // The sum is a chain of adds in row order, and the loads were too, one round trip to memory per
+    // row (192 us for windows of 512 rows): 32 rows are now read at once, the next 32 while these are added.
+    constexpr int U = 32;
+    float s = 0.f, v[U];
+    const int full = w.rows / U * U;
+    for (int r = 0; r < full; r += U) {
+#pragma unroll
+      for (int j = 0; j < U; j++) v[j] = p[(size_t)(r + j) * cols];
+#pragma unroll
+      for (int j = 0; j < U; j++) s += v[j];
+    }
+    for (int r = full; r < w.rows; r++) s += p[(size_t)r * cols];
     sums[c] = s;
   }
   __syncthreads();  // also orders the identity fill before the ranked writes
@@ -190,12 +200,16 @@ __device__ __forceinline__ uint32_t pk_symbol(float v) {
 }
 
 // ---- encode 4: scaling, symbols, histogram, scale_histogram.  One 1024-thread workgroup per
-// window. ----
-constexpr int HBINS = 8192;
+// window, so the latency of its loads and of LDS atomics bounds it.  Values are read eight at a time per
+// thread.  The counts of the QLOW lowest symbols, which nearly all values have, are kept per lane number
+// (a wave adds to 64 different banks; on one counter its atomics serialise) and summed at the end; the
+// rest, and every symbol past the first HBINS, are counted one counter per symbol. ----
+constexpr int HBINS = 8192, QLOW = 64, QU = 8;
 __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, PkWin* __restrict__ win, int cols,
                                                   uint16_t* __restrict__ syms, uint8_t* __restrict__ hdr_scratch,
                                                   uint32_t* __restrict__ pairs_scratch) {
   __shared__ uint32_t hist[HBINS];
+  __shared__ uint32_t low[QLOW * 64];
   __shared__ float red[32];
   __shared__ uint32_t ured[32];
   __shared__ uint32_t cnt_m;
@@ -205,10 +219,16 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
   uint16_t* sy = syms + (size_t)w.row0 * cols;
   // max over |x| < 1 (exact in any order), floor 1e-5
   float am = 0.00001f;
-  for (int i = tid; i < n; i += 1024) {
-    const float a = fabsf(v[i]);
-    if (a < 1.0f && a > am) am = a;
+  for (int i0 = tid; i0 < n; i0 += 1024 * QU) {
+    float a[QU];
+#pragma unroll
+    for (int j = 0; j < QU; j++) a[j] = i0 + 1024 * j < n ? fabsf(v[i0 + 1024 * j]) : 0.f;
+#pragma unroll
+    for (int j = 0; j < QU; j++)
+      if (a[j] < 1.0f && a[j] > am) am = a[j];
   }
+  for (int i = tid; i < HBINS; i += 1024) hist[i] = 0;
+  for (int i = tid; i < QLOW * 64; i += 1024) low[i] = 0;
   for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
   if (lane == 0) red[wid] = am;
   __syncthreads();
@@ -220,10 +240,19 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
   __syncthreads();
   const float inv = red[16];
   uint32_t ms = 0;
-  for (int i = tid; i < n; i += 1024) {
-    const uint32_t s = pk_symbol(v[i] * inv);
-    sy[i] = (uint16_t)s;
-    ms = ms > s ? ms : s;
+  for (int i0 = tid; i0 < n; i0 += 1024 * QU) {
+    float a[QU];
+#pragma unroll
+    for (int j = 0; j < QU; j++) a[j] = i0 + 1024 * j < n ? v[i0 + 1024 * j] : 0.f;
+#pragma unroll
+    for (int j = 0; j < QU; j++)
+      if (i0 + 1024 * j < n) {
+        const uint32_t s = pk_symbol(a[j] * inv);
+        sy[i0 + 1024 * j] = (uint16_t)s;
+        ms = ms > s ? ms : s;
+        if (s < QLOW) atomicAdd(&low[s * 64 + lane], 1u);
+        else if (s < HBINS) atomicAdd(&hist[s], 1u);
+      }
   }
   for (int o = 32; o > 0; o >>= 1) {
     const uint32_t t = __shfl_xor(ms, o);
@@ -232,18 +261,27 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
   if (lane == 0) ured[wid] = ms;
   if (tid == 0) cnt_m = 0;
   __syncthreads();
+  for (int s = wid; s < QLOW; s += 16) {
+    uint32_t c = low[s * 64 + lane];
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+    if (lane == 0) hist[s] = c;
+  }
   uint32_t max_sym = ured[0];
   for (int i = 1; i < 16; i++) max_sym = max_sym > ured[i] ? max_sym : ured[i];
-  // histogram in passes of HBINS symbols; the used symbols, in increasing order, with counts
+  __syncthreads();
+  // histogram in passes of HBINS symbols (the first is there); the used symbols, in increasing
+  // order, with counts
   uint32_t* pairs = pairs_scratch + (size_t)blockIdx.x * 4096 * 2;  // (symbol, count) then freq
   for (uint32_t base = 0; base <= max_sym; base += HBINS) {
-    for (int i = tid; i < HBINS; i += 1024) hist[i] = 0;
-    __syncthreads();
-    for (int i = tid; i < n; i += 1024) {
-      const uint32_t s = sy[i];
-      if (s >= base && s < base + HBINS) atomicAdd(&hist[s - base], 1u);
+    if (base > 0) {
+      for (int i = tid; i < HBINS; i += 1024) hist[i] = 0;
+      __syncthreads();
+      for (int i = tid; i < n; i += 1024) {
+        const uint32_t s = sy[i];
+        if (s >= base && s < base + HBINS) atomicAdd(&hist[s - base], 1u);
+      }
+      __syncthreads();
     }
-    __syncthreads();
     // compact the non-zero bins in order: per-thread chunks of 8 bins, exclusive scan of counts
     const int b0 = tid * 8;
     int nz = 0;
@@ -283,27 +321,28 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
   // the largest remainders (stable: lower index first on ties), residue to the last maximum.
   const uint64_t total = (uint64_t)n, rest = (uint64_t)(RANS_TOTAL - m);
   __syncthreads();
-  uint32_t* rem_rank = hist;  // reuse: rank of each symbol by remainder
+  // Each remainder (below n, so 32 bits) is taken once, not by every symbol that ranks itself
+  // against it: a 64-bit modulus is about 150 instructions.
+  uint32_t *rem = hist, *freq = hist + 4096;  // reuse
+  if (tid == 0) ured[0] = 0;
+  __syncthreads();
   for (int i = tid; i < m; i += 1024) {
-    const uint64_t ri = ((uint64_t)pairs[2 * i + 1] * rest) % total;
-    int rank = 0;
+    const uint64_t a = (uint64_t)pairs[2 * i + 1] * rest;
+    const uint32_t q = (uint32_t)(a / total);
+    rem[i] = (uint32_t)(a - q * total);
+    freq[i] = 1 + q;
+    atomicAdd(&ured[0], q);
+  }
+  __syncthreads();
+  const uint32_t deficit = (uint32_t)rest - ured[0];
+  for (int i = tid; i < m; i += 1024) {
+    const uint32_t ri = rem[i];
+    uint32_t rank = 0;
     for (int j = 0; j < m; j++) {
-      const uint64_t rj = ((uint64_t)pairs[2 * j + 1] * rest) % total;
+      const uint32_t rj = rem[j];
       rank += (rj > ri || (rj == ri && j < i)) ? 1 : 0;
     }
-    rem_rank[i] = rank;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t acc = 0;
-    for (int i = 0; i < m; i++) acc += (uint32_t)(((uint64_t)pairs[2 * i + 1] * rest) / total);
-    ured[0] = (uint32_t)rest - acc;  // deficit
-  }
-  __syncthreads();
-  const uint32_t deficit = ured[0];
-  for (int i = tid; i < m; i += 1024) {
-    const uint32_t q = (uint32_t)(((uint64_t)pairs[2 * i + 1] * rest) / total);
-    hist[4096 + i] = 1 + q + (rem_rank[i] < deficit ? 1u : 0u);
+    freq[i] += rank < deficit ? 1u : 0u;
   }
   __syncthreads();
   uint8_t* hdr = hdr_scratch + w.hdr;
@@ -311,15 +350,15 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
     int64_t tot = 0;
     int mi = 0;
     for (int i = 0; i < m; i++) {
-      tot += hist[4096 + i];
-      if (hist[4096 + i] >= hist[4096 + mi]) mi = i;
+      tot += freq[i];
+      if (freq[i] >= freq[mi]) mi = i;
     }
     while (tot < RANS_TOTAL) {
-      hist[4096 + mi]++;
+      freq[mi]++;
       tot++;
     }
-    while (tot > RANS_TOTAL && hist[4096 + mi] > 1) {
-      hist[4096 + mi]--;
+    while (tot > RANS_TOTAL && freq[mi] > 1) {
+      freq[mi]--;
       tot--;
     }
   }
@@ -330,7 +369,7 @@ __global__ __launch_bounds__(1024) void pk_quant(const float* __restrict__ x, Pk
     hdr[257] = (uint8_t)(m >> 8);
   }
   for (int i = tid; i < m; i += 1024) {
-    const uint32_t s = pairs[2 * i], f = hist[4096 + i];
+    const uint32_t s = pairs[2 * i], f = freq[i];
     uint8_t* p = hdr + 258 + 4 * i;
     p[0] = (uint8_t)s;
     p[1] = (uint8_t)(s >> 8);
