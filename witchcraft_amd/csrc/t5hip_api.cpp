@@ -1120,9 +1120,10 @@ void swap_lane(t5h_model* m, ExecLane& l) {
 
 // Batches of at least this many tokens (and two or more sequences) run as two halves, split at
 // the sequence boundary nearest T / 2, on two streams: one half's launches fill the CUs the
-// other's leave idle (tails of GEMM rounds, attention).  Measured per step, one lane vs two:
-// 71 k tokens (cfg4) 18.7 vs 17.5 ms, 16.8 k (cfg5) 4.29 vs 4.22 ms and 5.57 vs 5.35 ms with
-// hybrid numerics; 9.2 k and 4.4 k tokens are slower on two (2.48 vs 2.58 ms, 1.38 vs 1.42 ms).
+// other's leave idle (tails of GEMM rounds, attention).  Measured, one lane's time over two's:
+// 18 k tokens 1.00, 24 k 1.04, 36 k 1.06, 48 k 1.05, 54 k 0.975, 62 k 1.04, 71 k 0.985, 100 k 1.04,
+// 150 k 1.035 (which sizes lose follows the GEMM rounds of the halves, not T); hybrid numerics 1.01
+// at 17 k, 1.11 at 40 k, 1.10 at 70 k.  9.2 k and 4.4 k tokens were slower on two (0.96, 0.97).
 // Outputs are bit-identical (every output row is computed the same way: the GEMMs keep one K
 // order per output at any tile plan, attention is per sequence).
 constexpr int SPLIT_MIN_TOKENS = 16384;
