@@ -50,10 +50,10 @@ __device__ __forceinline__ void lds_load16(const void* base, uint32_t voff, uint
 // [0, NB / 2) are gate rows n0 .., blocks [NB / 2, NB) the up rows of the same columns.
 template <int EPI, int NB>
 __device__ __forceinline__ const char* wblock(const GemmArgs& p, int n0, int i) {
-  const _Float16* W = p.T0;
+  const void* W = p.W0;
   int n = n0 / 16 + i;
   if (EPI == EPI_GATED) {
-    W = i < NB / 2 ? p.T0 : p.T1;
+    W = i < NB / 2 ? p.W0 : p.W1;
     n = n0 / 16 + i % (NB / 2);
   }
   return reinterpret_cast<const char*>(W) + (size_t)n * (p.K / 32) * 1024;
@@ -437,7 +437,7 @@ hipError_t launch_tile_weights(const void* w, int wfmt, int N, int K, _Float16* 
 
 hipError_t launch_gemm(int epi, const GemmPlan& pl, const GemmArgs& a, hipStream_t s) {
   if (a.M <= 0) return hipSuccess;
-  if (!a.T0 || (epi == EPI_GATED && !a.T1)) return hipErrorInvalidValue;
+  if (!a.W0 || (epi == EPI_GATED && !a.W1)) return hipErrorInvalidValue;
   // whole tiles along N (128 weight rows at most: 64 columns of each matrix when gated) and whole
   // 128-wide K steps
   if (a.N % (epi == EPI_GATED ? 64 : 128) || a.K % 128) return hipErrorInvalidValue;

@@ -759,8 +759,8 @@ int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, con
     return T5H_OK;
   }
   if (norm_w) return fail(T5H_ERR_INVALID, "internal: fused norm requested on the batched GEMM path");
-  a.T0 = W.t;
-  a.T1 = W1 ? W1->t : nullptr;
+  a.W0 = W.t;
+  a.W1 = W1 ? W1->t : nullptr;
   t5k::GemmPlan plan = t5k::gemm_plan(epi, M, W.N * (W1 ? 2 : 1), W.K, m->cus);
   if (m->gemm_variant >= 0) plan.variant = m->gemm_variant;
   else if (epi == EPI_GATED && m->gated_mw8) plan.variant = t5k::GEMM_RING_128X128;  // 8 waves of 32 tokens
