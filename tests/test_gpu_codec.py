@@ -38,6 +38,32 @@ def test_residual_encode_bitexact(codec, N, D, K):
     assert np.array_equal(got, orc.residual_encode(emb, centers, assign))
 
 
+# The streamed form from 131,072 rows of 128 on, with a remainder of its 16-row workgroups, and sizes
+# beside it; buffers that start on any float.
+@pytest.mark.parametrize("N,D,K,shift", [(131072, 128, 300, 0), (131072 + 77, 128, 5, 3), (131072 - 1, 128, 300, 1),
+                                         (131072 + 1, 24, 9, 0)])
+def test_residual_encode_row_splits(codec, N, D, K, shift):
+    import torch
+    rng = np.random.default_rng(N + D)
+    emb, centers = (rng.normal(0, 0.1, (n, D)).astype(np.float32) for n in (N, K))
+    assign = rng.integers(0, K, N).astype(np.uint32)
+    dev = torch.device("cuda", 0)
+    e, c = (torch.zeros(x.size + shift, device=dev) for x in (emb, centers))
+    e[shift:] = torch.from_numpy(emb.ravel()).to(dev)
+    c[shift:] = torch.from_numpy(centers.ravel()).to(dev)
+    a = torch.from_numpy(assign.view(np.int32)).to(dev)
+    a[N // 2] = K  # no such centre: zero bytes and the flag
+    out = torch.full((N * D // 2 + 8,), 0x5a, dtype=torch.uint8, device=dev)
+    bad = torch.zeros(1, dtype=torch.int32, device=dev)
+    codec.residual_encode_device(e.data_ptr() + 4 * shift, N, c.data_ptr() + 4 * shift, K, a.data_ptr(), D,
+                                 out.data_ptr(), bad.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    got = out.cpu().numpy()
+    want = orc.residual_encode(emb, centers, assign)
+    want[N // 2] = 0
+    assert int(bad.item()) == 1
+    assert np.array_equal(got[:N * D // 2].reshape(N, D // 2), want) and np.all(got[N * D // 2:] == 0x5a)
+
+
 def test_residual_encode_edge_values(codec):
     t = codec.q4_compand_thresholds()
     specials = [0.0, -0.0, np.inf, -np.inf, np.nan, 1e-30, -1e-30, 3.4e38, -3.4e38, 1.0, -1.0, 0.25, -0.25]

@@ -81,6 +81,72 @@ __global__ __launch_bounds__(256) void residual_encode_kernel(const float* __res
   *reinterpret_cast<uint32_t*>(out + (size_t)row * (D / 2) + 4 * g) = word;
 }
 
+// Byte offset into the heap of thresholds (T[1] = t[7], children of T[i] at 2 i and 2 i + 1, so
+// T[8 .. 15] = t[0], t[2], ..) after one comparison: 4 (2 i + (r >= T[i])).  NaN compares false.
+__device__ __forceinline__ uint32_t q4_step(uint32_t at, float r, float t) { return 2 * at + (r >= t ? 4u : 0u); }
+
+// 4 x the code of r.  t1, t2, t3: the heap's first three entries, from registers.
+__device__ __forceinline__ uint32_t q4_code4(float r, const float* heap, float t1, float t2, float t3) {
+  const bool up = r >= t1;
+  uint32_t at = q4_step(up ? 12u : 8u, r, up ? t3 : t2);
+  at = q4_step(at, r, *reinterpret_cast<const float*>(reinterpret_cast<const char*>(heap) + at));
+  at = q4_step(at, r, *reinterpret_cast<const float*>(reinterpret_cast<const char*>(heap) + at));
+  return at - 64;
+}
+
+// 128-d rows by the hundred thousand, bound by the embeddings' one pass through memory: 32 lanes a
+// row, four values a lane, so a wave's loads are contiguous, and two rows a thread, both rows' loads
+// in flight before the first is used.  Embeddings and codes are non-temporal, which leaves the L2s to
+// the centres.  1,000,003 rows, 16,384 centres: 134 us with a thread per eight values -> 116 us
+// (5.0 TB/s; a large copy reaches 5.06 on the same card); one row a thread 172, three 124, four 123,
+// plain code stores 119.
+constexpr int kEncU = 2;  // rows per thread; a workgroup takes 8 kEncU rows
+// From here on it is the faster one whether or not the rows are in the caches: 131,072 rows 19.6 us
+// warm and 21.2 from memory against 18.8 and 18.9, 100,000 rows 13.1 and 16.1 against 13.5 and 14.1.
+constexpr size_t kEncStreamRows = 131072;
+__global__ __launch_bounds__(256) void residual_encode_stream_kernel(const float* __restrict__ emb,
+                                                                     const float* __restrict__ centers,
+                                                                     const uint32_t* __restrict__ assign, int N,
+                                                                     int K, Q4Ladder lad, uint8_t* __restrict__ out,
+                                                                     unsigned* __restrict__ bad) {
+  constexpr int D = 128;
+  typedef f4v f4u __attribute__((aligned(4)));
+  __shared__ float heap[16];
+  if (threadIdx.x >= 1 && threadIdx.x < 16) {
+    const int i = threadIdx.x, level = 31 - __clz(i);
+    heap[i] = lad.t[((2 * (i - (1 << level)) + 1) << (3 - level)) - 1];
+  }
+  __syncthreads();
+  const int c = threadIdx.x & 31;
+  const size_t first = (size_t)blockIdx.x * (8 * kEncU) + (threadIdx.x >> 5);
+  const float t1 = lad.t[7], t2 = lad.t[3], t3 = lad.t[11];
+  uint32_t a[kEncU];
+  f4v e[kEncU], m[kEncU];
+#pragma unroll
+  for (int u = 0; u < kEncU; u++) a[u] = assign[min(first + 8 * u, (size_t)N - 1)];
+#pragma unroll
+  for (int u = 0; u < kEncU; u++)
+    e[u] = __builtin_nontemporal_load(
+        reinterpret_cast<const f4u*>(emb + min(first + 8 * u, (size_t)N - 1) * D + 4 * c));
+#pragma unroll
+  for (int u = 0; u < kEncU; u++)
+    m[u] = *reinterpret_cast<const f4u*>(centers + (size_t)(a[u] < (uint32_t)K ? a[u] : 0u) * D + 4 * c);
+#pragma unroll
+  for (int u = 0; u < kEncU; u++) {
+    const size_t row = first + 8 * u;
+    if (row >= (size_t)N) break;
+    uint32_t q[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[j] = q4_code4(e[u][j] - m[u][j], heap, t1, t2, t3);
+    uint32_t w = (q[0] << 2) | (q[1] >> 2) | (q[2] << 10) | (q[3] << 6);  // byte j / 2: value j in the high nibble
+    if (a[u] >= (uint32_t)K) {
+      w = 0;
+      if (c == 0) atomicOr(bad, 1u);
+    }
+    __builtin_nontemporal_store((uint16_t)w, reinterpret_cast<uint16_t*>(out + row * (D / 2) + 2 * c));
+  }
+}
+
 // from_companded_q4_bytes: one thread per 4 code bytes -> 8 floats.
 __global__ __launch_bounds__(256) void residual_decode_kernel(const uint8_t* __restrict__ codes, size_t nbytes,
                                                               Q4Table tab, float* __restrict__ out) {
@@ -483,6 +549,12 @@ namespace t5k {
 hipError_t launch_residual_encode(const float* emb, const float* centers, const uint32_t* assign, int N, int D,
                                   int K, const Q4Ladder& lad, uint8_t* out, unsigned* bad, hipStream_t s) {
   if (N <= 0) return hipSuccess;
+  // Non-temporal code stores want whole 128-byte lines: a wave's two rows.
+  if (D == 128 && (size_t)N >= kEncStreamRows && ((uintptr_t)out & 127) == 0) {
+    hipLaunchKernelGGL(residual_encode_stream_kernel, dim3((unsigned)(((size_t)N + 8 * kEncU - 1) / (8 * kEncU))),
+                       dim3(256), 0, s, emb, centers, assign, N, K, lad, out, bad);
+    return hipGetLastError();
+  }
   const size_t threads = (size_t)N * (D / 8);
   hipLaunchKernelGGL(residual_encode_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, emb, centers,
                      assign, N, D, K, lad, out, bad);
