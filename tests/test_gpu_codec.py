@@ -148,7 +148,8 @@ def test_matmul_t_q4_within_f32_summation_bound(codec, M, N, D):
 # the streaming kernel's passes and edges: one column short of and past a 32-column tile, a lane's
 # four columns cut at 1..3, one row in the last pass, the smallest and a long stream, both store kinds
 Q4_STREAM_SHAPES = [(33, 512), (1, 513), (16, 514), (64, 515), (32, 4095), (65, 4097), (50, 9001), (17, 65537),
-                    (33, 65536), (100, 30752)]
+                    (33, 65536), (100, 30752),
+                    (13, 163840), (7, 327680), (43, 65568)]  # non-temporal: rows past M in either half of a 16-row block
 
 
 @pytest.mark.parametrize("M,N", Q4_STREAM_SHAPES)

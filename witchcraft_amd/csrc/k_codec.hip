@@ -421,19 +421,40 @@ __global__ __launch_bounds__(256, 2) void matmul_t_q4_split_kernel(const float* 
         }
       }
   };
+  // Whole tiles only when non-temporal (N % 32 == 0): lanes lr and lr ^ 8 trade a half tile, so that a
+  // store instruction writes 8 rows of 128 bytes instead of 16 of 64 (32 x 1,048,576 57.6 -> 55.1 us).
+  const bool upper = lr >= 8;
   int soff[MB];
 #pragma unroll
-  for (int i = 0; i < MB; i++) soff[i] = ((16 * i + lr) * N + 4 * lg) * 4;
+  for (int i = 0; i < MB; i++)
+    soff[i] = NT ? ((16 * i + (lr & 7)) * N + (upper ? 16 : 0) + 4 * lg) * 4 : ((16 * i + lr) * N + 4 * lg) * 4;
   auto store = [&](int t, const f4v (&acc)[MB][2]) {
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc((void*)(C + (size_t)t * 32), (short)0, 0x7fffffff, kBufDword3);
+    if constexpr (NT) {
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        f4v c0, c1;  // rows 16 i + lr % 8 and + 8, columns 16 .. 31 on the upper lanes
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const float x = upper ? acc[i][0][j] : acc[i][1][j];
+          const float y = __int_as_float(
+              __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+          c0[j] = upper ? y : acc[i][0][j];
+          c1[j] = upper ? acc[i][1][j] : y;
+        }
+        if (16 * i + (lr & 7) < M) __builtin_amdgcn_raw_buffer_store_b128(c0, rs, soff[i], 0, kBufNt);
+        if (16 * i + 8 + (lr & 7) < M) __builtin_amdgcn_raw_buffer_store_b128(c1, rs, soff[i] + 32 * N, 0, kBufNt);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < MB; i++) {
       const bool row_ok = 16 * i + lr < M;
 #pragma unroll
       for (int nb = 0; nb < 2; nb++)
         if (row_ok && 32 * t + 16 * nb + 4 * lg + 3 < N)
-          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, NT ? kBufNt : 0);
+          __builtin_amdgcn_raw_buffer_store_b128(acc[i][nb], rs, soff[i] + 64 * nb, 0, 0);
       if (t >= nfull && row_ok)
 #pragma unroll
         for (int nb = 0; nb < 2; nb++) {  // the last tile: N may end inside a lane's four columns
@@ -584,9 +605,9 @@ hipError_t launch_matmul_t_q4(const float* A, const uint8_t* codes, const Q4Tabl
     const int wgs = std::min(2 * num_cus_codec(), (N + 127) / 128);
     // Scores as non-temporal stores where every store fills whole 128-byte lines and the scores outgrow
     // what the L2s would keep for a reader anyway: twice the bytes of the codes at 32 rows, they otherwise
-    // evict the codes of the next tiles (32 x 1,048,576 76 -> 63 us, 16 x 262,144 17.9 -> 16.3, 32 x
-    // 65,536 12.4 -> 11.7).  Rows that start inside a line lose, each half line going out by itself (32 x
-    // 1,048,575 78 -> 131 us).
+    // evict the codes of the next tiles (with 64-byte stores 32 x 1,048,576 76 -> 63 us, 16 x 262,144
+    // 17.9 -> 16.3, 32 x 65,536 12.4 -> 11.7).  Rows that start inside a line lose, each half line going
+    // out by itself (32 x 1,048,575 78 -> 131 us).
     const bool nt = N % 32 == 0 && ((uintptr_t)C & 127) == 0 && (size_t)M * N * 4 >= (size_t)8 << 20;
     // T5H_Q4_SCORE_F32=1 keeps the f32-MFMA stream (measurement and tests)
     static const bool f32_only = [] {
