@@ -195,6 +195,30 @@ def test_small_model_last_key_tile_of_a_long_sequence(small, tiles):
         _check_batch(gpu, ora, ids, cu)
 
 
+@pytest.mark.parametrize("base,step", [(2.0 ** 27, 16), (2.0 ** 27 + 2.0 ** 26, 16)])
+def test_small_model_scores_a_step_of_f32_apart(enc_mod, base, step):
+    """Relative-position biases so large that one step of f32 is 16: far keys score one step above near
+    ones, in a later key tile for the first queries, so the softmax reference must move (e^16 is no
+    f16).  q.k has a deviation of about 1 here, under half a step, so every score is base or
+    base + step exactly and the oracle's softmax is the same one."""
+    cfg = synth.small_config()
+    name = "encoder.block.0.layer.0.SelfAttention.relative_attention_bias.weight"
+    shape = (cfg["relative_attention_num_buckets"], cfg["num_heads"])
+    old = synth._normal(17, name, shape, cfg["d_model"] ** -0.5).tobytes()
+    bias = np.full(shape, base, np.float32)
+    bias[[15, 31]] += step  # the last bucket of either direction: 113 tokens away or more
+    img = synth.make_model(cfg, seed=17)
+    assert img.count(old) == 1
+    img = img.replace(old, bias.tobytes())
+    gpu, ora = enc_mod.T5EncoderModel.from_gguf(img, cfg), orc.OracleModel(img, cfg)
+    try:
+        cu = np.cumsum([0, 300, 513, 192]).astype(np.int32)
+        ids = np.random.default_rng(5).integers(1, cfg["vocab_size"], size=int(cu[-1])).astype(np.uint32)
+        _check_batch(gpu, ora, ids, cu)
+    finally:
+        gpu.close()
+
+
 def test_small_model_max_length_sequence(small):
     cfg, _, gpu, ora = small
     ids = np.random.default_rng(2).integers(1, cfg["vocab_size"], size=2048).astype(np.uint32)

@@ -178,16 +178,17 @@ __device__ __forceinline__ h8 v_operand(const _Float16* Vb, int c, int vo) {
 //
 // The reference max moves only when needed.  A query's scores lie in two lanes (the two key
 // halves of each 8-key group), so its tile max is one permlane32 swap away; the reference
-// m_run is moved to the running max, and O and l rescaled, only when some query's tile max
-// exceeds m_run by more than 14 / log2(e), i.e. m_lim (always on the first tile, where both are -inf), so
-// every P = 2^((s - m_run) log2e) stays at most 2^14, well inside f16.  Same result up to
-// rounding: P and l carry the same factor, divided out at the end, and m_run is a score
-// already seen, so l >= 1.  A rescale on every tile measured slower.  l sums the f16 P that the
+// m_run is moved to the running max, and O and l rescaled, only when the exponent of some P =
+// 2^(s log2e - m_run log2e) would exceed 14 (always on the first tile, where m_run is -inf), so
+// that P stays well inside f16.  The test takes that exponent as the products below round it: a
+// limit in units of the score, m_run + 14 / log2(e), is a whole step of f32 off where the scores
+// are beyond 2^26, and let P overflow.  Same result up to rounding: P and l carry the same factor,
+// divided out at the end, and m_run is a score already seen.  A rescale on every tile measured slower.  l sums the f16 P that the
 // P.V product uses; it is kept per lane (this lane's keys) and reduced across the two lanes of
 // a query only at the end.
 template <bool FULL, bool MASK>
 __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* Vb, const float* Bsb, LaneOfs& lo,
-                                          const h8 (&qf)[4], bool qv, int k0, int L, float& m_run, float& m_lim,
+                                          const h8 (&qf)[4], bool qv, int k0, int L, float& m_run, float& mb,
                                           float& l_run, f16v (&o)[2]) {
   constexpr int NS = FULL ? 2 : 1;  // 32-key halves with keys < L
   const int h = (threadIdx.x >> 5) & 1;
@@ -241,23 +242,22 @@ __device__ __forceinline__ void attn_tile(const _Float16* Ksb, const _Float16* V
   for (int kb = 0; kb < NS; kb++)
 #pragma unroll
     for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[kb][r]);
-  // mx is the max of this lane's half of the keys; some lane of a query exceeds m_lim exactly if
-  // the query's max does, so the lanes only meet in the branch.  m_lim is +inf for queries past
-  // L, so that whatever those rows hold cannot change when the valid queries rescale: the result
-  // stays independent of the batch around the sequence.
-  if (__builtin_amdgcn_ballot_w64(mx > m_lim)) {
+  // mx is the max of this lane's half of the keys; some lane of a query exceeds the limit exactly if
+  // the query's max does, so the lanes only meet in the branch.  mb = -m_run log2e, or -inf for
+  // queries past L (P = 0), so that whatever those rows hold cannot change when the valid queries
+  // rescale: the result stays independent of the batch around the sequence.
+  if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(mx, LOG2E, mb) > 14.f)) {
     mx = max_xor32(mx);  // finite: key k0 < L is valid
     // the rescale of O sits in a branch of its own, so the accumulators keep their registers
     const float m_new = fmaxf(m_run, mx);
     // 1 where the max did not move, 0 on the first tile (O and l are still 0 there)
     const float corr = __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E);
     m_run = m_new;
-    m_lim = qv ? m_new + 14.f / LOG2E : INFINITY;
+    mb = qv ? -m_new * LOG2E : -INFINITY;
     l_run *= corr;
 #pragma unroll
     for (int db = 0; db < 2; db++) o[db] *= corr;
   }
-  const float mb = -m_run * LOG2E;
 
   // P = 2^(S log2e - m_run log2e) in f16; O^T[d][query] += V^T[d][keys] . P^T[keys][query] over
   // the 16-key steps of the valid halves, the P^T operand of step c being registers
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
   };
   static_assert(LOADS == 5, "the wait below counts five loads per tile");
 
-  float m_run = -INFINITY, m_lim = qi < L ? -INFINITY : INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, mb = qi < L ? INFINITY : -INFINITY, l_run = 0.f;
   f16v o[2];
 #pragma unroll
   for (int db = 0; db < 2; db++)
@@ -469,13 +469,13 @@ __global__ __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(3))) v
     if (!decltype(act)::value) return;
     const int k0 = t * KT;
     if (!decltype(tail)::value) {
-      attn_tile<true, false>(cur.k, cur.v, cur.b, lofs, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
+      attn_tile<true, false>(cur.k, cur.v, cur.b, lofs, qf, qi < L, k0, L, m_run, mb, l_run, o);
       return;
     }
     LaneOfs lt = lofs;  // (three variants that redefine one set of offsets would spill)
-    if (!last) attn_tile<true, false>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
-    else if (L - k0 > 32) attn_tile<true, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
-    else attn_tile<false, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, m_lim, l_run, o);
+    if (!last) attn_tile<true, false>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, mb, l_run, o);
+    else if (L - k0 > 32) attn_tile<true, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, mb, l_run, o);
+    else attn_tile<false, true>(cur.k, cur.v, cur.b, lt, qf, qi < L, k0, L, m_run, mb, l_run, o);
   };
   // The Q loads complete before tile 0, which is peeled off the loop, so that the loop body (whose
   // steps are never the last tile) carries a single tile variant and no wait on them.
