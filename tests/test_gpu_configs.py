@@ -361,6 +361,49 @@ def test_hybrid_bf16_weights_differ_from_hybrid(xtr_hybrid):
         assert rel(outs[mode], refs[mode]) < rel(outs[mode], refs[other]), mode
 
 
+def test_bf16_weights_out_of_memory_leaves_the_handle(xtr):
+    """t5h_set_numerics(HYBRID_BF16) makes two copies of the dense weights.  With room for one only it
+    reports the error, gives the first one back, and the handle serves its old numerics and, with
+    memory again, the new ones."""
+    import torch
+    from witchcraft_amd._lib import T5H_ERR_NOMEM, T5HError
+    from witchcraft_amd.encoder import T5EncoderModel
+    cfg, img, ref, _ = xtr
+    D, inner = cfg["d_model"], cfg["num_heads"] * cfg["d_kv"]
+    copy = 2 * cfg["num_layers"] * (4 * D * inner + D * cfg["d_ff"])
+    ids = np.random.default_rng(3).integers(1, cfg["vocab_size"], size=200).astype(np.uint32)
+    cu = np.array([0, 200], np.int32)
+    free = lambda: torch.cuda.mem_get_info(0)[0]  # noqa: E731
+    gpu = T5EncoderModel.from_gguf(img, cfg)
+    try:
+        want, _ = gpu.encode_packed(ids, cu)
+        torch.cuda.empty_cache()
+        fill = []
+        for _ in range(4):  # the first large block takes less than its size from the free count
+            if free() > 1.7 * copy:
+                fill.append(torch.empty(free() - 3 * copy // 2, dtype=torch.uint8, device="cuda:0"))
+        before = free()
+        if not 1.1 * copy < before < 1.9 * copy:
+            pytest.skip(f"{before} bytes free beside the filler")
+        for _ in range(2):
+            with pytest.raises(T5HError) as e:
+                gpu.set_numerics(2)
+            assert e.value.code == T5H_ERR_NOMEM
+            assert free() > before - copy // 2
+        got, _ = gpu.encode_packed(ids, cu)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        del fill
+        torch.cuda.empty_cache()
+        gpu.set_numerics(2)
+        got, _ = gpu.encode_packed(ids, cu)
+        ref.set_numerics(2)
+        want, _ = ref.encode_packed(ids, cu)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    finally:
+        ref.set_numerics(0)
+        gpu.close()
+
+
 @pytest.mark.parametrize("layout,mode,variant",
                          [("hybrid", 1, orc.VARIANT_HYBRID), ("hybrid", 2, orc.VARIANT_HYBRID_BF16),
                           ("q4k", 2, orc.VARIANT_HYBRID_BF16)],

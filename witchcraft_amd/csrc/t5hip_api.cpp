@@ -14,6 +14,7 @@
 #include <mutex>
 #include <stdlib.h>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/t5hip.h"
@@ -628,6 +629,7 @@ int build_tiled(t5h_model* m, const std::vector<Linear*>& ls, void** buf) {
   for (const Linear* L : ls) need += align256((size_t)L->N * L->K * 2);
   if (hipMalloc(buf, need) != hipSuccess) {
     *buf = nullptr;
+    (void)hipGetLastError();  // or the next launch would report it
     return fail(T5H_ERR_NOMEM, "weight operand allocation of " + std::to_string(need) + " bytes failed");
   }
   size_t off = 0;
@@ -1924,7 +1926,8 @@ int t5h_ffn_block(t5h_model* m, int32_t layer, const float* x, int32_t T, float*
 namespace {
 // The dense linears of T5H_NUMERICS_HYBRID_BF16 (q/k/v or the fused qkv, o, wo): F32/F16 ones
 // point at their arena copy of the truncated weights; Q4_K ones are expanded once into bfw
-// (dequantized exactly, truncated to bf16, stored as f16 [N][K]).  Synchronous.
+// (dequantized exactly, truncated to bf16, stored as f16 [N][K]).  Synchronous.  On failure the
+// handle is as it was: both allocations belong to `o` until they are complete.
 int build_bf16_layers(t5h_model* m) {
   if (!m->layers_bf.empty()) return T5H_OK;
   std::vector<Layer> lb = m->layers;
@@ -1940,17 +1943,28 @@ int build_bf16_layers(t5h_model* m) {
     dense.push_back(&Ly.o);
     dense.push_back(&Ly.wo);
   }
+  struct Owner {
+    hipStream_t stream;
+    void *w = nullptr, *t = nullptr;
+    ~Owner() {
+      if (!w && !t) return;
+      (void)hipStreamSynchronize(stream);  // launches that write them may be under way
+      if (w) (void)hipFree(w);
+      if (t) (void)hipFree(t);
+    }
+  } o{m->stream};
   size_t need = 0;
   for (const Linear* L : dense)
     if (L->fmt == WF_Q4K) need += align256((size_t)L->N * L->K * 2);
-  if (need && hipMalloc(&m->bfw, need) != hipSuccess) {
-    m->bfw = nullptr;
+  if (need && hipMalloc(&o.w, need) != hipSuccess) {
+    o.w = nullptr;
+    (void)hipGetLastError();  // or the next launch would report it
     return fail(T5H_ERR_NOMEM, "bf16 weight allocation of " + std::to_string(need) + " bytes failed");
   }
   size_t off = 0;
   for (Linear* L : dense) {
     if (L->fmt == WF_Q4K) {
-      _Float16* dst = (_Float16*)((uint8_t*)m->bfw + off);
+      _Float16* dst = (_Float16*)((uint8_t*)o.w + off);
       HIP_OK(t5k::launch_q4k_dequant_bf16_f16(L->w, (size_t)L->N * L->K / QK_K, dst, m->stream));
       off += align256((size_t)L->N * L->K * 2);
       L->w = dst;
@@ -1961,8 +1975,10 @@ int build_bf16_layers(t5h_model* m) {
     L->fmt = WF_F16;
   }
   int rc;
-  if ((rc = build_tiled(m, dense, &m->twb))) return rc;
+  if ((rc = build_tiled(m, dense, &o.t))) return rc;
   HIP_OK(hipStreamSynchronize(m->stream));
+  m->bfw = std::exchange(o.w, nullptr);
+  m->twb = std::exchange(o.t, nullptr);
   m->layers_bf = std::move(lb);
   return T5H_OK;
 }
