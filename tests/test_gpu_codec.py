@@ -209,6 +209,23 @@ def test_matmul_t_q4_shape_errors(codec):
         codec.matmul_t_q4(np.zeros((2, 128), np.float32), np.zeros((3, 32), np.uint8))
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+def test_matmul_t_q4_finds_a_nonfinite_value_anywhere(codec, M):
+    """The value that sends a pass of query rows to the f32 kernel may sit in any row and column: an
+    infinity at the corners of every 16-row block gives scores of infinity with the sign of the
+    decoded value it meets, and the other rows stay finite."""
+    rng = np.random.default_rng(M)
+    codes = rng.integers(0, 256, (600, 64)).astype(np.uint8)
+    r = orc.residual_decode(codes, 128)
+    for row in sorted({0, M // 2, M - 1} | set(range(15, M, 16)) | set(range(16, M, 16))):
+        for col in (0, 3, 124, 127):
+            a = _unit_rows(M, 128, rng)
+            a[row, col] = np.inf
+            got = codec.matmul_t_q4(a, codes)
+            assert np.array_equal(got[row], np.copysign(np.float32(np.inf), r[:, col])), (row, col)
+            assert np.isfinite(np.delete(got, row, 0)).all(), (row, col)
+
+
 def test_matmul_t_q4_nonfinite_query(codec):
     """The streaming shape runs on bf16 MFMAs with both operands split in three parts, which
     cannot carry infinities (inf times parts of both signs would give NaN); a query block with a

@@ -345,10 +345,15 @@ __global__ __launch_bounds__(256, 2) void matmul_t_q4_split_kernel(const float* 
     pt[x] = make_uint4(h0 | (h1 << 16), m0 | (m1 << 16), l0 | (l1 << 16), 0u);
     // Non-finite values, and finite ones of magnitude >= 0x7f7f8000 (which round to a bf16
     // infinity in split3, so x - inf would give NaN), take the f32 kernel.
+    // 16 bytes a load, all unconditional (row M - 1 stands for rows past it) and so all in flight at
+    // once: one value a load under a row test took a trip to memory each, 32 x 4,096 8.1 -> 6.3 us.
     int nf = 0;
-    for (int e = threadIdx.x; e < 16 * MB * D; e += 256) {
-      const int r = e / D;
-      if (r < M && !(fabsf(A[(size_t)r * D + (e - r * D)]) < __uint_as_float(0x7f7f8000u))) nf = 1;
+#pragma unroll
+    for (int j = 0; j < 2 * MB; j++) {
+      const int e = threadIdx.x + 256 * j;
+      const float4 v = *reinterpret_cast<const float4*>(A + (size_t)min(e / (D / 4), M - 1) * D + 4 * (e % (D / 4)));
+      const float big = __uint_as_float(0x7f7f8000u);
+      if (!(fabsf(v.x) < big) || !(fabsf(v.y) < big) || !(fabsf(v.z) < big) || !(fabsf(v.w) < big)) nf = 1;
     }
     if (nf) bad = 1;  // every writer stores 1
   }
@@ -598,8 +603,8 @@ hipError_t launch_matmul_t_q4(const float* A, const uint8_t* codes, const Q4Tabl
                               int D, hipStream_t s) {
   if (M <= 0 || N <= 0) return hipSuccess;
   // A long stream of 128-d codes takes the streaming kernels in passes of 32 query rows, at any N:
-  // split kernel / tiled kernel below: 32 x 1,000 8.8 / 9.9 us, 32 x 131,071 18.8 / 30, 50 x 200,000
-  // 34 / 77, 32 x 1,048,575 78 / 226, 1,000 x 16,384 73 / 98.  (Scores may start on any f32: 16-byte
+  // split kernel / tiled kernel below: 32 x 1,000 6.2 / 9.4 us, 48 x 16,384 6.7 / 10.4, 48 x 200,000
+  // 26 / 64, 32 x 1,048,575 59 / 204, 1,000 x 16,384 69 / 97.  (Scores may start on any f32: 16-byte
   // buffer stores need 4-byte alignment only.)
   const bool aligned = ((uintptr_t)A & 15) == 0 && ((uintptr_t)codes & 15) == 0;
   const int mb = M <= 16 ? 1 : 2, passes = M <= 16 ? 1 : (M + 31) / 32;
