@@ -39,9 +39,11 @@ def test_residual_encode_bitexact(codec, N, D, K):
 
 
 # The streamed form from 131,072 rows of 128 on, with a remainder of its 16-row workgroups, and sizes
-# beside it; buffers that start on any float.
+# beside it; buffers that start on any float; cached and non-temporal embeddings (from 524,288 rows or
+# 8,192 centres on).
 @pytest.mark.parametrize("N,D,K,shift", [(131072, 128, 300, 0), (131072 + 77, 128, 5, 3), (131072 - 1, 128, 300, 1),
-                                         (131072 + 1, 24, 9, 0)])
+                                         (131072 + 1, 24, 9, 0), (131072 + 5, 128, 8192, 1), (140001, 128, 8191, 2),
+                                         (524288, 128, 7, 3), (524287, 128, 7, 0)])
 def test_residual_encode_row_splits(codec, N, D, K, shift):
     import torch
     rng = np.random.default_rng(N + D)
@@ -85,6 +87,21 @@ def test_residual_encode_edge_values(codec):
     # and against the scalar quantizer, value by value
     codes = np.stack([got >> 4, got & 15], axis=-1).reshape(-1)
     assert [int(c) for c in codes[: vals.size]] == [orc.compand_q4(v) for v in vals]
+
+
+@pytest.mark.parametrize("K", [1, 8192])
+def test_residual_encode_edge_values_streamed(codec, K):
+    """The same values at a size that takes the streamed form, in every column and either row of a
+    thread, with cached and with non-temporal embeddings."""
+    specials = [0.0, -0.0, np.inf, -np.inf, np.nan, 1e-30, -1e-30, 3.4e38, -3.4e38, 1.0, -1.0, 0.25, -0.25]
+    t = codec.q4_compand_thresholds().astype(np.float32)
+    vals = np.concatenate([np.array(specials, np.float32), t, np.nextafter(t, np.float32(np.inf)),
+                           np.nextafter(t, np.float32(-np.inf))])
+    N, D = 131072, 128  # 58 values: successive rows start at different ones
+    emb = np.resize(vals, N * D).reshape(N, D)
+    got = codec.residual_to_q4_bytes(emb, np.zeros((K, D), np.float32), np.zeros(N, np.uint32))
+    codes = np.stack([got >> 4, got & 15], axis=-1).reshape(-1)
+    assert np.array_equal(codes, np.resize(np.array([orc.compand_q4(v) for v in vals], np.uint8), N * D))
 
 
 def test_residual_encode_rejects_bad_assignment(codec):

@@ -96,14 +96,19 @@ __device__ __forceinline__ uint32_t q4_code4(float r, const float* heap, float t
 
 // 128-d rows by the hundred thousand, bound by the embeddings' one pass through memory: 32 lanes a
 // row, four values a lane, so a wave's loads are contiguous, and two rows a thread, both rows' loads
-// in flight before the first is used.  Embeddings and codes are non-temporal, which leaves the L2s to
-// the centres.  1,000,003 rows, 16,384 centres: 134 us with a thread per eight values -> 116 us
-// (5.0 TB/s; a large copy reaches 5.06 on the same card); one row a thread 172, three 124, four 123,
-// plain code stores 119.
+// in flight before the first is used.  Codes are non-temporal, and so are the embeddings (NT) where
+// that pays: rows that outgrow the 256 MB last-level cache, or centres that fill an XCD's 4 MB L2 and
+// are kept there.  Otherwise rows that a caller has just written come faster from that cache: 400,000
+// rows, 64 centres 33 us plain, 44 non-temporal (45 both when not cached), 300,000 rows, 8,192 centres
+// 35.7 and 34.4, 16,384 centres 40.6 and 37.0.  1,000,003 rows, 16,384 centres: 134 us with a thread
+// per eight values -> 116 us (5.0 TB/s; a large copy reaches 5.06 on the same card); one row a thread
+// 172, three 124, four 123, plain code stores 119.
 constexpr int kEncU = 2;  // rows per thread; a workgroup takes 8 kEncU rows
+constexpr size_t kEncNtBytes = (size_t)256 << 20, kEncNtCentres = (size_t)4 << 20;
 // From here on it is the faster one whether or not the rows are in the caches: 131,072 rows 19.6 us
 // warm and 21.2 from memory against 18.8 and 18.9, 100,000 rows 13.1 and 16.1 against 13.5 and 14.1.
 constexpr size_t kEncStreamRows = 131072;
+template <bool NT>
 __global__ __launch_bounds__(256) void residual_encode_stream_kernel(const float* __restrict__ emb,
                                                                      const float* __restrict__ centers,
                                                                      const uint32_t* __restrict__ assign, int N,
@@ -125,9 +130,10 @@ __global__ __launch_bounds__(256) void residual_encode_stream_kernel(const float
 #pragma unroll
   for (int u = 0; u < kEncU; u++) a[u] = assign[min(first + 8 * u, (size_t)N - 1)];
 #pragma unroll
-  for (int u = 0; u < kEncU; u++)
-    e[u] = __builtin_nontemporal_load(
-        reinterpret_cast<const f4u*>(emb + min(first + 8 * u, (size_t)N - 1) * D + 4 * c));
+  for (int u = 0; u < kEncU; u++) {
+    const f4u* p = reinterpret_cast<const f4u*>(emb + min(first + 8 * u, (size_t)N - 1) * D + 4 * c);
+    e[u] = NT ? __builtin_nontemporal_load(p) : *p;
+  }
 #pragma unroll
   for (int u = 0; u < kEncU; u++)
     m[u] = *reinterpret_cast<const f4u*>(centers + (size_t)(a[u] < (uint32_t)K ? a[u] : 0u) * D + 4 * c);
@@ -579,8 +585,12 @@ hipError_t launch_residual_encode(const float* emb, const float* centers, const 
   if (N <= 0) return hipSuccess;
   // Non-temporal code stores want whole 128-byte lines: a wave's two rows.
   if (D == 128 && (size_t)N >= kEncStreamRows && ((uintptr_t)out & 127) == 0) {
-    hipLaunchKernelGGL(residual_encode_stream_kernel, dim3((unsigned)(((size_t)N + 8 * kEncU - 1) / (8 * kEncU))),
-                       dim3(256), 0, s, emb, centers, assign, N, K, lad, out, bad);
+    const dim3 grid((unsigned)(((size_t)N + 8 * kEncU - 1) / (8 * kEncU)));
+    const bool nt = (size_t)N * D * 4 >= kEncNtBytes || (size_t)K * D * 4 >= kEncNtCentres;
+    if (nt) hipLaunchKernelGGL((residual_encode_stream_kernel<true>), grid, dim3(256), 0, s, emb, centers, assign, N, K,
+                               lad, out, bad);
+    else hipLaunchKernelGGL((residual_encode_stream_kernel<false>), grid, dim3(256), 0, s, emb, centers, assign, N, K,
+                            lad, out, bad);
     return hipGetLastError();
   }
   const size_t threads = (size_t)N * (D / 8);
