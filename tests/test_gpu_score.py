@@ -73,7 +73,10 @@ def test_matmul_t_vs_oracle(score, M, N, D, bf16_b):
 # the streaming kernel's passes and edges: one column short of and past a 32-column tile, a lane's
 # four columns cut at 1..3, one row in the last pass, the last row count of its range, both store kinds
 STREAM_SHAPES = [(33, 512), (1, 513), (16, 514), (64, 515), (32, 4095), (65, 4097), (17, 65537), (33, 65536),
-                 (128, 16416)]
+                 (128, 16416),
+                 # two to four passes that share the workgroups, with more tiles than waves; 33 to 48 rows
+                 # where the tiled kernel takes them and where it does not
+                 (49, 40000), (65, 40001), (97, 33000), (48, 40000), (33, 40001), (48, 66000), (40, 100000)]
 
 
 @pytest.mark.parametrize("bf16_b", [False, True])

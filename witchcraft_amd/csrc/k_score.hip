@@ -737,14 +737,27 @@ hipError_t launch_matmul_t(const float* A, const float* B, float* C, int M, int 
   if (tiles_n * tiles_m > 0x7fffffffL) return hipErrorInvalidValue;
   const dim3 grid((unsigned)(tiles_n * tiles_m));
   const bool vec = D % 4 == 0 && aligned16(A) && aligned16(B) && aligned16(C);
-  // Few rows of A against a long B: the persistent streaming kernel, 2 workgroups per CU, in passes of
-  // 32 rows.  Streaming kernel / tiled kernel: 32 x 1,000 8.3 / 9.5 us, 50 x 16,384 8.5 / 15.7,
-  // 50 x 200,000 50 / 64, 64 x 200,001 60 / 84, 128 x 4,096 9.3 / 15.7; from 256 rows on B is read again
-  // once too often (256 x 16,384 19.5 / 19.1, 1,000 x 50,000 215 / 182).
+  // Few rows of A against a long B: the persistent streaming kernel in passes of 32 rows.  The passes
+  // share two workgroups per CU, in whole groups of 8, so that the same columns meet in one XCD's L2 in
+  // every pass; with two per CU for each pass they ran one after the other and read B again (33 x 50,000
+  // 18.8 -> 15.0 us, 80 x 200,000 67 -> 54, 112 x 1,048,576 519 -> 382).  Streaming kernel / tiled
+  // kernel: 32 x 1,000 5.9 / 8.9 us, 48 x 16,384 6.5 / 12.2, 64 x 65,536 15.7 / 18.6, 64 x 200,000 47 / 59,
+  // 128 x 4,096 6.1 / 15.3; from 256 rows on the tiled kernel (256 x 16,384 19.5 / 19.1, 1,000 x 50,000
+  // 215 / 182 before the passes shared).
   const bool rows16 = D % 4 == 0 && aligned16(A) && aligned16(B);
-  if (rows16 && D == 128 && M <= 128 && N >= 512 && 32L * N * 4 < (1L << 31)) {
+  bool stream = rows16 && D == 128 && M <= 128 && N >= 512 && 32L * N * 4 < (1L << 31);
+  // 33 to 48 rows are three of the tiled kernel's row blocks but two passes: it takes them where its
+  // rounds of 256 columns per CU, 13 us each, cost less than the streaming kernel's of 128, 6.1 us each
+  // behind 3 us (40,000 columns 13.4 / 15.2 us, 80,000 25 / 20), and where B outgrows the last-level cache,
+  // which the two passes then drift apart in (40 x 1,048,576 214 / 224).
+  if (stream && mb == 3 && vec && N % 4 == 0) {
+    const long cus = num_cus(), wide = (N + 256 * cus - 1) / (256 * cus), narrow = (N + 128 * cus - 1) / (128 * cus);
+    stream = 13.0 * wide > 3 + 6.1 * narrow && (size_t)N * D * 4 < (size_t)384 << 20;
+  }
+  if (stream) {
     const int passes = mb == 1 ? 1 : (M + 31) / 32;
-    const dim3 g((unsigned)std::min<long>(2L * num_cus(), (N + 127) / 128), (unsigned)passes);
+    const long per = passes == 1 ? 2L * num_cus() : std::max(8L, 2L * num_cus() / passes / 8 * 8);
+    const dim3 g((unsigned)std::min<long>(per, (N + 127) / 128), (unsigned)passes);
     // scores past the caches as they are written: a store of whole 128-byte lines, and more of them than
     // the L2s would hold for a reader (16 x 262,144 34.9 -> 33.4 us, 32 x 1,048,576 140.5 -> 137; a row
     // that starts inside a line loses: see matmul_t_q4's rule)
