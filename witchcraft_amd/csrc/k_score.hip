@@ -354,15 +354,20 @@ __global__ __launch_bounds__(256) void matmul_argmax_kernel(const float* __restr
 // product is hi hi + hi lo + lo hi, each exact in the f32 accumulator: 3 f16 MFMAs for 16 f32
 // ones.  What is dropped (lo lo and the r terms) is at most 2^-21 |a b| per product, without a
 // common sign over the 128 products; the f32 accumulation takes 24 steps where the f32 MFMAs take
-// 32.  (131,072 normal rows x 16,384 normal columns, three seeds: 0, 0 and 2 rows other than in
-// 64 bits, against 1, 0 and 2 on f32 MFMAs.)
+// 32.  So the scores compared are nearer to 64 bits than on f32 MFMAs: winning scores 1.0e-7 off (2-norm;
+// largest 4 to 7e-7) against 1.7e-7 (7 to 11e-7), over normal, clustered and all-positive rows and columns
+// of one size or spread over 50 and 10,000 times; 1.1 to 1.3e-7 against 1.4 to 1.6e-7 on heavy tails.
 //  * Rows of A: each scaled by its own power of two (an argmax over the row does not change) and
 //    held in registers for the whole run, 32 RBL rows per wave on 32x32x16 MFMAs.
 //  * Columns of B: 64 or 128 at a time through double-buffered LDS, split once per workgroup on
-//    the way in, all by one power of two set from the first columns.  A column must then stay
-//    inside f16's precise range: largest |b s| in [2^3, 2^15], or all zeros.
-//  * A row or column outside those ranges, infinite or NaN makes the workgroup redo its rows on
-//    f32 MFMAs (argmax_rows_f32), so such inputs give what they gave before.
+//    the way in, by one power of two set from the first columns, whose largest value comes to the
+//    middle of f16's precise range.  A column whose largest |b s| lies outside [2^3, 2^15] takes a
+//    power of two of its own, which is taken out of its products again, exactly, before they are
+//    compared (cscale).  4,096 x 16,384: 275 us, one column at the end 16 times larger 275, empty
+//    columns in front 275, sizes over three decades 495; 2,460 to 2,740 when such columns sent all
+//    rows to the f32 MFMAs.
+//  * A column 2^60 off the first ones, a row beyond 2^-87 .. 2^123, an infinity or a NaN makes the
+//    workgroup redo its rows on f32 MFMAs (argmax_rows_f32), so such inputs give what they gave there.
 // The 8 waves of a workgroup hold 8 / WN row groups; the WN waves of a group take 1 / WN of a
 // chunk's columns each, for inputs with too few rows to fill the chip.
 // 131,072 x 16,384: 5.03 ms on f32 MFMAs (109 TFLOP/s) -> 1.28-1.40 ms (390-430); 4,096 x 4,096:
@@ -500,6 +505,10 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
   __shared__ float4 lds[LDS4];  // chunks [2][PARTS][PART] h8, or argmax_rows_f32's
   __shared__ float red[8];
   __shared__ int redo[2];  // by barrier parity: a flag is rewritten only after every thread has read it
+  // what each column's products are multiplied by, and whether any factor of a buffer has ever been
+  // other than 1, so that the products need a look at them
+  __shared__ __attribute__((aligned(16))) float cscale[2][COLS];
+  __shared__ int scaled[2];
   h8* Bs = reinterpret_cast<h8*>(lds);
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, lr = lane & 31, lg = lane >> 5;
@@ -511,41 +520,68 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
   const int c0 = tid >> 5, k4 = tid & 31;
   float4 st[NL];
   auto gload = [&](int n0) {  // also past the last chunk: unconditional, so nothing waits for it early
+    const int first = min(n0, N - 1);  // 64-bit on the scalar unit, 32-bit offsets inside the chunk
+    const char* base = reinterpret_cast<const char*>(B) + (size_t)first * (4 * D);
 #pragma unroll
     for (int j = 0; j < NL; j++)
-      st[j] = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(B) +
-                                               ((uint32_t)min(n0 + c0 + 16 * j, N - 1) * (4u * D) + 16u * k4));
+      st[j] = *reinterpret_cast<const float4*>(base + ((uint32_t)min(c0 + 16 * j, N - 1 - first) * (4u * D) + 16u * k4));
   };
   gload(0);
-  {  // one power of two for every column: the first chunk's largest magnitude comes to [2^12, 2^13)
+  for (int i = tid; i < 2 * COLS; i += 512) (&cscale[0][0])[i] = 1.f;
+  {  // one power of two for every column: the first chunk's largest magnitude comes to [2^9, 2^10)
     float m = 0.f;
 #pragma unroll
     for (int j = 0; j < NL; j++) m = fmaxf(m, max4abs(BF16B ? trunc_bf16(st[j]) : st[j]));
     m = max_xor32(max32(m));
     if (lane == 0) red[wave] = m;
-    if (tid == 0) redo[0] = redo[1] = 0;
+    if (tid == 0) redo[0] = redo[1] = scaled[0] = scaled[1] = 0;
   }
   __syncthreads();
   float bmax = red[0];
 #pragma unroll
   for (int i = 1; i < 8; i++) bmax = fmaxf(bmax, red[i]);
-  const uint32_t be = float_exp(bmax);
-  if (be < 40 || be > 250) bad = true;  // zeros, tiny, huge, infinite
-  const float bs = pow2_bits(bad ? 127 : 127 + 12 + 127 - be);
+  const bool empty = bmax == 0.f;  // all columns of the first chunk: then as for values of size 1
+  const uint32_t be = empty ? 127 : float_exp(bmax);
+  if (be < 40 || be > 250) bad = true;  // tiny, huge, infinite
+  const uint32_t bse = bad ? 127 : 127 + 9 + 127 - be;  // exponent of the common power of two
+  const float bs = pow2_bits(bse);
+  int own = 0;  // bit buf: this wave has factors other than 1 in cscale[buf]
   // 16-byte chunk k / 8 of column c sits at chunk (k / 8) ^ (c % 16): the operand reads below (32
   // columns x one chunk) and these stores (one column, 16 chunks) hit every bank once
   const int at0 = (c0 * 16 + ((k4 >> 1) ^ c0)) * 2 + (k4 & 1);
   auto lstore = [&](int buf) {
+    uint32_t u[NL];   // largest magnitude of the thread's values: infinities and NaNs compare above every finite one
+    bool odd = false;  // wave-uniform: some column outside the range of the common power of two
 #pragma unroll
     for (int j = 0; j < NL; j++) {
       const float4 v = BF16B ? trunc_bf16(st[j]) : st[j];
-      // largest magnitude as an integer: infinities and NaNs compare above every finite value
-      const uint32_t u = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
-                             max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
-      const float m = __uint_as_float(u) * bs;
+      u[j] = max(max(__float_as_uint(v.x) & 0x7fffffffu, __float_as_uint(v.y) & 0x7fffffffu),
+                 max(__float_as_uint(v.z) & 0x7fffffffu, __float_as_uint(v.w) & 0x7fffffffu));
+      const float m = __uint_as_float(u[j]) * bs;
       // a column is a wave half: some lane reaches 2^3 or every lane is zero
-      const unsigned long long big = __builtin_amdgcn_ballot_w64(m >= 8.f), any = __builtin_amdgcn_ballot_w64(u != 0);
-      bad |= !(m <= 32768.f) || ((uint32_t)big == 0 && (uint32_t)any != 0) || (big >> 32 == 0 && any >> 32 != 0);
+      const unsigned long long big = __builtin_amdgcn_ballot_w64(m >= 8.f), any = __builtin_amdgcn_ballot_w64(u[j] != 0);
+      odd |= __builtin_amdgcn_ballot_w64(!(m <= 32768.f)) != 0 || ((uint32_t)big == 0 && (uint32_t)any != 0) ||
+             (big >> 32 == 0 && any >> 32 != 0);
+    }
+    if (__builtin_expect(odd || (own >> buf & 1), 0)) {
+#pragma unroll
+      for (int j = 0; j < NL; j++) {
+        const float top = max32(__uint_as_float(min(u[j], 0x7f800000u)));  // the column's largest; NaN as infinity
+        const int e = (int)float_exp(top), k = (int)be - e;  // by 2^k it comes to the first chunk's size
+        const bool out = top != 0.f && !(top * bs >= 8.f && top * bs <= 32768.f);
+        const bool far = out && (e < 1 || e == 255 || k < -60 || k > 60);
+        bad |= far;
+        const int by = out && !far ? k : 0;
+        const float f = pow2_bits(127 + by);
+        st[j] = make_float4(st[j].x * f, st[j].y * f, st[j].z * f, st[j].w * f);
+        if (k4 == 0) cscale[buf][c0 + 16 * j] = pow2_bits(127 - by);
+      }
+      own = odd ? own | 1 << buf : own & ~(1 << buf);
+      if (lane == 0) scaled[buf] = 1;
+    }
+#pragma unroll
+    for (int j = 0; j < NL; j++) {
+      const float4 v = BF16B ? trunc_bf16(st[j]) : st[j];
       h4 hi, lo;
       _Float16 h, l;
       split_f16(v.x, bs, h, l); hi[0] = h; lo[0] = l;
@@ -599,6 +635,7 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
   if (bad) redo[0] = 1;
   __syncthreads();
   auto multiply = [&](int buf, int n0) {
+    const int factors = __builtin_amdgcn_readfirstlane(scaled[buf]);
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) {
       f16v acc[RBL];
@@ -630,6 +667,19 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
         for (int rb = 0; rb < RBL; rb++)
           acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh[ks & 1], ah[rb][ks], acc[rb], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+      }
+      if (__builtin_expect(factors, 0)) {
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+          const float4 c = *reinterpret_cast<const float4*>(&cscale[buf][32 * (cb0 + cb) + 2 * i + 4 * lg]);
+#pragma unroll
+          for (int rb = 0; rb < RBL; rb++) {
+            acc[rb][i] *= c.x;
+            acc[rb][i + 1] *= c.y;
+            acc[rb][i + 2] *= c.z;
+            acc[rb][i + 3] *= c.w;
+          }
+        }
       }
       // lane: row lr of the block, columns 8 (i / 4) + 4 lg + i % 4 of the 32, ascending in i, so
       // the first of equal scores is kept by "greater" over chunks and a descending search inside
@@ -800,7 +850,7 @@ hipError_t launch_matmul_argmax(const float* A, const float* B, uint32_t* out, i
   if (M <= 0) return hipSuccess;
   if (N <= 0 || D < 0) return hipErrorInvalidValue;
   const bool vec = D % 4 == 0 && aligned16(A) && aligned16(B);
-  if (vec && D == 128 && N < (1 << 23)) {  // byte offsets of B fit 32 bits
+  if (vec && D == 128) {
     // Rows per workgroup (one workgroup per CU at a time): a shorter tile re-splits B more often per
     // row but fills the chip with fewer rows.  Times of one round over 4,096 columns: 512 rows 279
     // us, 256 rows 195, 128 rows 110, 64 rows 80; the least rounds x time is taken (16,384 x 4,096:
