@@ -160,7 +160,8 @@ def test_matmul_argmax_many_rows_vs_oracle(score, bf16_b):
 # rows x columns around the four tile heights (64, 128, 256 and 512 rows per workgroup on 256 CUs)
 # and around the 64- and 128-column chunks
 @pytest.mark.parametrize("bf16_b", [False, True])
-@pytest.mark.parametrize("M,N", [(1, 2), (63, 64), (65, 129), (16385, 65), (32769, 127), (65537, 63), (131073, 70)])
+@pytest.mark.parametrize("M,N", [(1, 2), (63, 64), (65, 129), (16385, 65), (32769, 127), (65537, 63), (131073, 70),
+                                 (65536, 2), (49000, 33), (65535, 129)])
 def test_matmul_argmax_tiles_vs_oracle(score, M, N, bf16_b):
     a, b = _data(M, N, 128, seed=M + N)
     got = score.matmul_argmax(a, b, bf16_b=bf16_b)

@@ -853,10 +853,13 @@ hipError_t launch_matmul_argmax(const float* A, const float* B, uint32_t* out, i
   if (vec && D == 128) {
     // Rows per workgroup (one workgroup per CU at a time): a shorter tile re-splits B more often per
     // row but fills the chip with fewer rows.  Times of one round over 4,096 columns: 512 rows 279
-    // us, 256 rows 195, 128 rows 110, 64 rows 80; the least rounds x time is taken (16,384 x 4,096:
-    // 80 us on 64 rows, 97 on 128, 166 on 256, 258 on 512, 233 on the f32 kernel below).
+    // us, 256 rows 190, 128 rows 110, 64 rows 80; the least rounds x time is taken (16,384 x 4,096:
+    // 80 us on 64 rows, 97 on 128, 166 on 256, 258 on 512, 233 on the f32 kernel below).  256 rows are
+    // eight waves of 32, each on all columns: four pairs of 64 rows that halve the columns read every row
+    // of A twice, which bounds few columns (65,536 rows x 64 columns 11.4 us, by pairs 15.8, the f32
+    // kernel 13.9; x 1,024 55 and 59; x 16,384 702 and 694).
     const long cus = num_cus();
-    const double cost[4] = {279, 195, 110, 80};
+    const double cost[4] = {279, 190, 110, 80};
     int v = 0;
     double best = 1e30;
     for (int i = 0; i < 4; i++) {
@@ -877,7 +880,7 @@ hipError_t launch_matmul_argmax(const float* A, const float* B, uint32_t* out, i
   } while (0)
     switch (v) {
       case 0: T5K_AMS(2, 1); break;
-      case 1: T5K_AMS(2, 2); break;
+      case 1: T5K_AMS(1, 1); break;
       case 2: T5K_AMS(1, 2); break;
       default: T5K_AMS(1, 4); break;
     }
