@@ -634,8 +634,7 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
   }
   if (bad) redo[0] = 1;
   __syncthreads();
-  auto multiply = [&](int buf, int n0) {
-    const int factors = __builtin_amdgcn_readfirstlane(scaled[buf]);
+  auto multiply = [&](int buf, int n0, int factors) {
 #pragma unroll
     for (int cb = 0; cb < CB; cb++) {
       f16v acc[RBL];
@@ -703,6 +702,7 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
   // runs beside the other's MFMAs.
   const int nchunks = (N + COLS - 1) / COLS;
   bool f32 = redo[0];  // workgroup-uniform
+  int factors = __builtin_amdgcn_readfirstlane(scaled[0]);
   for (int ch = 0; ch < nchunks && !f32; ch++) {
     const int buf = ch & 1;
     if (wave < 4) {
@@ -710,7 +710,7 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
       gload((ch + 2) * COLS);
       __builtin_amdgcn_sched_barrier(0);
     }
-    multiply(buf, ch * COLS);
+    multiply(buf, ch * COLS, factors);
     if (wave >= 4) {
       lstore(buf ^ 1);
       gload((ch + 2) * COLS);
@@ -718,6 +718,7 @@ __global__ __launch_bounds__(512, 2) void matmul_argmax_split_kernel(const float
     if (bad) redo[(ch + 1) & 1] = 1;
     __syncthreads();
     f32 = redo[(ch + 1) & 1];
+    factors = __builtin_amdgcn_readfirstlane(scaled[(ch + 1) & 1]);
   }
   if (f32) {
     for (int r = wg_r0; r < min(wg_r0 + wg_rows, M); r += 256) {
