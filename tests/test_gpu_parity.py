@@ -234,7 +234,8 @@ def test_xtr_cfg2_sample_vs_oracle(xtr):
 
 def test_xtr_cfg4_lengths_vs_oracle(xtr):
     """Sequences of the bulk config's upper range (400-512 tokens, 7-8 key tiles) in a ~2,300-token
-    batch: full GEMM tiles, thin tails and long attention rows, every sequence against the oracle."""
+    batch: direct GEMM tiles, the last ones part-filled, and long attention rows, every sequence against
+    the oracle."""
     cfg, _, gpu, ora = xtr
     ids, cu = synth.ragged_batch(5, 400, 512, cfg["vocab_size"], seed=15)
     assert cu[-1] > 1500
@@ -470,8 +471,8 @@ def test_hybrid_layout_f32_attention_weights(enc_mod):
 
 
 def test_xtr_hybrid_layout_large_batch_vs_oracle(enc_mod):
-    """cfg5's layout at XTR-base size, with a batch (~2,000 tokens) large enough for the full
-    4-wave x 128-row tiles and thin tails of the f16-weight GEMMs (q/k/v/o/wo)."""
+    """cfg5's layout at XTR-base size, with a batch (~2,000 tokens) large enough for the direct tiles of
+    q/k/v and o, part-filled at its end."""
     cfg = dict(synth.XTR_BASE)
     img = synth.make_model(cfg, seed=41, layout="hybrid")
     gpu = enc_mod.T5EncoderModel.from_gguf(img, cfg)
@@ -595,9 +596,8 @@ def test_sequence_output_independent_of_batch_neighbours(xtr):
 
 
 def _handles_by_tail(enc_mod, img, cfg):
-    """Handles on one model with the batched GEMM's thin tail tiles off (T5H_GEMM_TAIL=0),
-    forced to 16 (1) and to 32 (2) token rows per math wave for the last row of full tiles, and
-    with full tiles of 48 tokens per math wave and thin tails of 32 (T5H_GEMM_MB=3, "mb3")."""
+    """Handles on one model whose batched GEMMs all take one direct tile: 256 tokens high
+    (T5H_GEMM_TAIL=0), 64 (1), 128 (2) and 192 (T5H_GEMM_MB=3, "mb3")."""
     import os
     hs = {}
     for v in ("0", "1", "2", "mb3"):
@@ -613,8 +613,9 @@ def _handles_by_tail(enc_mod, img, cfg):
 
 @pytest.mark.parametrize("layout", ["q4k", "hybrid"])
 def test_thin_tail_tiles_are_bit_identical(enc_mod, xtr, layout):
-    """Thin tail tiles run the same K order per output as full tiles: every tile plan gives the
-    same bits, through all 12 layers (Q4_K and f16 weights), with the chosen plan in between."""
+    """Tiles of every height run the same K order per output: 64, 128 and 192 tokens give the bits of 256,
+    through all 12 layers (Q4_K and f16 weights), and so does the plan's own choice.  (The name is from
+    when a launch could end in thinner tiles.)"""
     cfg, img, gpu, _ = xtr
     if layout == "hybrid":
         img = synth.make_model(cfg, seed=3, layout="hybrid")
@@ -802,8 +803,9 @@ def test_tile_width_does_not_change_bits(enc_mod, xtr):
             h.close()
 
 
-# token counts over which the planner goes through every form and tile, each a few tokens past or
-# short of whole tiles
+# Token counts (one lane each) at which, between them, every launch (QKV, O, gate|up, wo, projection)
+# takes every form and tile that the planner ever gives it for this model on 256 CUs, a few tokens past
+# or short of whole tiles; O and wo take the two-step ring at 10,753 only
 @pytest.mark.parametrize("layout", ["q4k", "hybrid"])
 def test_gemm_forms_are_bit_identical(enc_mod, xtr, layout):
     """The ring and direct GEMM forms take K in one order: the planner's choice at every size gives
@@ -814,7 +816,7 @@ def test_gemm_forms_are_bit_identical(enc_mod, xtr, layout):
         gpu = enc_mod.T5EncoderModel.from_gguf(img, cfg)
     hs = [_handle_with_env(enc_mod, img, cfg, T5H_GEMM_TAIL=t) for t in ("0", "1")]
     try:
-        for T in (65, 127, 161, 255, 300, 513, 700, 1100, 1700, 2100, 3300, 4700, 6300, 9001, 13000):
+        for T in (65, 127, 161, 255, 300, 513, 700, 1100, 1700, 2100, 3300, 4700, 6300, 9001, 10753, 13000):
             cu = np.unique(np.r_[0:T:500, T]).astype(np.int32)
             ids = np.random.default_rng(T).integers(1, cfg["vocab_size"], size=T).astype(np.uint32)
             got, _ = gpu.encode_packed(ids, cu)
