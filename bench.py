@@ -13,6 +13,7 @@ Prints ONE JSON line.  Extra fields:
                    hybrid-dequant + fbgemm numerics in C) on a bounded sample of the same
                    workload, batch-1 per sequence as the reference runs it;
   kernels       -- per-kernel-class averages from the same event timing;
+  configs       -- (cfg2) cfg4 and cfg5 in brief; their whole records go to stderr;
   query         -- (cfg2) the cfg3 query regime: p50 / p95 latency over 1,000 queries cycling
                    8 model replicas, and its dominant GEMV against the HBM roofline.
 """
@@ -46,6 +47,40 @@ WORKLOADS = {
 
 def log(msg: str) -> None:
     print(msg, file=sys.stderr, flush=True)
+
+
+def short(x):
+    """x with its floats at 5 significant digits."""
+    if isinstance(x, dict):
+        return {k: short(v) for k, v in x.items()}
+    if isinstance(x, (list, tuple)):
+        return [short(v) for v in x]
+    return float(f"{x:.5g}") if isinstance(x, float) else x
+
+
+def brief(r: dict) -> dict:
+    """A further workload's part of the line; its whole record goes to stderr."""
+    b = {k: r[k] for k in ("workload", "value", "unit", "ms_per_step", "steps", "tokens_per_step", "numerics") if k in r}
+    b["roofline"] = {k: r["roofline"][k] for k in ("kernel", "bound", "achieved", "peak", "unit", "frac", "avg_launch_us")
+                     if k in r["roofline"]}
+    if "cpu_baseline" in r:
+        b["cpu_baseline"] = {k: r["cpu_baseline"][k] for k in ("value", "unit", "cores") if k in r["cpu_baseline"]}
+    return b
+
+
+def emit(line: dict) -> None:
+    """The JSON line: the headline in full, the further workloads (`configs`, the query's kernel table)
+    in brief and floats at 5 digits, so that it stays a few kilobytes long: a reader that keeps only
+    the end of the output must find all of it."""
+    out = short(line)
+    for name, r in out.get("configs", {}).items():
+        log(f"[bench] record {name}: " + json.dumps(r, separators=(",", ":")))
+        out["configs"][name] = brief(r)
+    if "query" in out:
+        log("[bench] record query: " + json.dumps(out["query"], separators=(",", ":")))
+        out["query"].pop("kernels", None)
+    out.update({k: line[k] for k in ("value", "ms_per_step") if k in line})
+    print(json.dumps(out, separators=(",", ":")), flush=True)
 
 
 def cpu_info() -> dict:
@@ -319,7 +354,7 @@ def query_bench(args) -> None:
         "roofline": q["roofline"], "cpu_baseline": q["cpu_baseline"], "kernels": q["kernels"],
         "query_bytes": q["query_bytes"], "query_floor_us": q["query_floor_us"],
     }
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 PEAK_F32_MFMA_TFLOPS = 157.3  # MI355X dense f32 MFMA
@@ -481,7 +516,7 @@ def score_bench(args) -> None:
                           "peak_tflops": PEAK_F32_MFMA_TFLOPS, **kmeans},
         "cpu_baseline": base,
     }
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 def embed_bench(args) -> None:
@@ -549,7 +584,7 @@ def embed_bench(args) -> None:
                    "note": "host buffers in and out: PCIe copies inside the timed region"},
         "cpu_baseline": base, "kernels": kernels,
     }
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 def codec_bench(args) -> None:
@@ -606,7 +641,7 @@ def codec_bench(args) -> None:
         "encode_call_wall_ms": sorted(wall)[len(wall) // 2] * 1e3,
         "cpu_baseline": base,
     }
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 NUMERICS = {"default": 0, "hybrid": 1, "hybrid_bf16": 2}
@@ -1001,7 +1036,7 @@ def main() -> None:
         line["configs"] = extra
     if w == "cfg2" and not args.no_query:
         line["query"] = run_query(args, img if args.seed == 0 else None)
-    print(json.dumps(line), flush=True)
+    emit(line)
 
 
 def run_query_counter_pass(args) -> None:
