@@ -357,7 +357,6 @@ def query_bench(args) -> None:
     emit(line)
 
 
-PEAK_F32_MFMA_TFLOPS = 157.3  # MI355X dense f32 MFMA
 
 
 def _event_time(torch, fn, reps: int) -> float:
@@ -452,7 +451,7 @@ def score_bench(args) -> None:
     estep()
     es = _event_time(torch, estep, args.steps)
     e_bytes = N * D * 4 + N * 4 + N * D // 2
-    enc = {"kernel": "residual_encode_kernel (threshold ladder)", "avg_launch_us": es * 1e6,
+    enc = {"kernel": "residual_encode_stream_kernel (threshold ladder)", "avg_launch_us": es * 1e6,
            "rows_per_s": N / es, "bytes_per_launch": e_bytes, "gbs": e_bytes / es / 1e9,
            "hbm_frac": e_bytes / es / 1e9 / PEAK_HBM_GBS}
     log(f"[bench] residual encode [{N}x{D}]: {es * 1e6:.1f} us, {e_bytes / es / 1e9:.0f} GB/s")
@@ -471,7 +470,7 @@ def score_bench(args) -> None:
         ks = _event_time(torch, kstep, max(3, args.steps // 4))
         tf = 2.0 * km * kk * D / ks / 1e12
         kmeans["bf16_b" if bf else "f32"] = {"avg_launch_us": ks * 1e6, "tflops": tf,
-                                             "mfma_frac": tf / PEAK_F32_MFMA_TFLOPS}
+                                             "mfma_frac": (2 if bf else 3) * tf / PEAK_F16_TFLOPS}
         log(f"[bench] kmeans assign {'bf16_b' if bf else 'f32'} [{km}x{kk}]: {ks * 1e3:.2f} ms, {tf:.1f} TFLOP/s")
 
     base = None
@@ -512,8 +511,9 @@ def score_bench(args) -> None:
                      "traffic": traffic, "bytes_per_launch": bytes_per_launch, "avg_launch_us": avg_s * 1e6},
         "q4_scoring": q4,
         "residual_encode": enc,
-        "kmeans_assign": {"kernel": "matmul_argmax_kernel", "M": km, "N": kk, "D": D, "bound": "mfma",
-                          "peak_tflops": PEAK_F32_MFMA_TFLOPS, **kmeans},
+        "kmeans_assign": {"kernel": "matmul_argmax_split_kernel (f16 parts: 3 x v_mfma_f32_32x32x16_f16 per block, "
+                                    "2 with bf16 B)", "M": km, "N": kk, "D": D, "bound": "mfma",
+                          "peak_tflops": PEAK_F16_TFLOPS, **kmeans},
         "cpu_baseline": base,
     }
     emit(line)
