@@ -190,8 +190,11 @@ int t5h_matmul_t(int32_t hip_device, const float* a, int32_t M, const float* b, 
                  int32_t bf16_b, float* c);
 /* matmul_argmax_batched (src/lib.rs:187-208, k-means assignment at :235,1330):
  * out[i] = argmax_j A[i] . B[j], the first (smallest) j on ties as candle's argmax (0 when no
- * score exceeds -inf).  N > 0.  Same buffers and numerics as t5h_matmul_t, no [M][N]
- * intermediate. */
+ * score exceeds -inf).  N > 0.  Same buffers as t5h_matmul_t, no [M][N] intermediate.  Scores are
+ * compared in f32 and lie within its summation bound, but not on the same bits as t5h_matmul_t's:
+ * at D = 128 a product comes from two f16 parts per operand, at most 2^-21 of it dropped (rows or
+ * columns whose sizes leave that form's range, or are not finite, on f32 MFMAs), so columns whose
+ * scores differ by less than that rounding may be ordered either way. */
 int t5h_matmul_argmax(int32_t hip_device, const float* a, int32_t M, const float* b, int32_t N,
                       int32_t D, int32_t bf16_b, uint32_t* out);
 /* The same on device buffers of the current device, enqueued on `stream` (a hipStream_t;
@@ -227,8 +230,10 @@ int t5h_residual_decode(int32_t hip_device, const uint8_t* codes, int32_t N, int
 int t5h_residual_decode_device(const uint8_t* d_codes, int32_t N, int32_t D, float* d_out, void* stream);
 /* Search-time residual scores without materialising the residuals (src/lib.rs:676-680,734-735):
  * C[M][N] = A[M][D] . from_companded_q4_bytes(codes)[N][D]^T, D % 4 == 0, within the f32
- * summation bound D * 2^-23 * sum |a||r| of the f32 product (query-sized A against many rows
- * runs on bf16 MFMAs with both operands split in three parts; non-finite queries on f32). */
+ * summation bound D * 2^-23 * sum |a||r| of the f32 product (D = 128, N >= 512 runs on bf16
+ * MFMAs with both operands split in three parts, six of the nine part products taken and the
+ * other three below 2^-25 of a product; non-finite queries on f32).  Scores are stored in whole
+ * 128-byte lines when N % 32 == 0 and C starts on 128 bytes, the fastest form for large N. */
 int t5h_matmul_t_q4(int32_t hip_device, const float* a, int32_t M, const uint8_t* codes, int32_t N, int32_t D,
                     float* c);
 int t5h_matmul_t_q4_device(const float* d_a, int32_t M, const uint8_t* d_codes, int32_t N, int32_t D, float* d_c,

@@ -17,8 +17,8 @@
 // steps of 64.  A goes from global memory straight to the wave's registers (no other wave needs it),
 // one contiguous 1 KiB load per operand, one step ahead; the weight step, which all four waves
 // read, goes global -> LDS without registers into the other half of a double buffer.  Bound at
-// large M (gate|up, MB = 3, counters): MFMA busy 57% at the 1.83 GHz that power leaves, three waves
-// per SIMD waiting to issue 57% of their cycles, vector-memory return path busy 94%.
+// large M (gate|up, MB = 3, counters): MFMA busy 57% at the 1.7 GHz that power leaves, three waves
+// per SIMD waiting to issue 57% of their cycles, vector-memory return path busy 93%.
 //
 // Ring form (ring_gemm_kernel): both operands through an LDS ring several steps deep, for launches
 // with so few tiles that a step waits on memory: tiles of 32 x 64 to 128 x 128 tokens x rows.  A
