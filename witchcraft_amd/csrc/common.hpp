@@ -64,7 +64,6 @@ __host__ __device__ __forceinline__ size_t tiled_index(size_t m, size_t k, size_
 
 struct GemmArgs {
   const _Float16* A;  // [Mpad][K] f16 in operand order (tiled_index), Mpad >= roundup(M, 512)
-  int lda;            // unused (A's row length is K)
   const void* W0;  // [N][K] weights (Q4_K blocks row-major along K, or f16); launch_gemm: the f16
                    // operand as launch_tile_weights lays it out
   const void* W1;  // second weight for EPI_GATED

@@ -433,9 +433,10 @@ __global__ __launch_bounds__(256, 2) void matmul_t_q4_split_kernel(const float* 
       }
   };
   // Whole tiles only when non-temporal (N % 32 == 0): lanes lr and lr ^ 8 trade a half tile, so that a
-  // store instruction writes 8 rows of 128 bytes instead of 16 of 64.  Medians of alternating runs:
-  // 32 x 65,536 11.2 -> 10.7 us, 50 x 200,000 33.6 -> 32.4, 32 x 1,048,576 60.5 -> 58.9; 16 x 1,048,576
-  // 42.4 -> 42.8, 8 x 1,048,576 40.6 -> 40.4.
+  // store instruction writes 8 rows of 128 bytes instead of 16 of 64.  Medians of alternating runs
+  // when this came in: 32 x 65,536 11.2 -> 10.7 us, 50 x 200,000 33.6 -> 32.4, 32 x 1,048,576 60.5 -> 58.9;
+  // 16 x 1,048,576 42.4 -> 42.8, 8 x 1,048,576 40.6 -> 40.4.  With the query check above: 32 x 1,048,576
+  // 53 us on cached codes, 59 on new ones.
   const bool upper = lr >= 8;
   int soff[MB];
 #pragma unroll

@@ -712,11 +712,10 @@ int rec_stride(const t5h_model* m, int T) { return use_gemv(m, T) ? NORM_REC_GEM
 // C = A . W^T (+ epilogue).  norm_w: on the GEMV path the operand is T5LayerNorm(m->w.x) with
 // this weight, computed inside the kernel (A is then unused); callers pass it only when
 // use_gemv() holds.  nl: folded norm (fold_norm() holds), on either path.
-int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, const _Float16* A, int lda,
-         int M, void* out, int ldo, int n_off = 0, const float* norm_w = nullptr, const NormLink* nl = nullptr) {
+int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, const _Float16* A, int M,
+         void* out, int ldo, int n_off = 0, const float* norm_w = nullptr, const NormLink* nl = nullptr) {
   GemmArgs a{};
   a.A = A;
-  a.lda = lda;
   a.W0 = W.w;
   a.W1 = W1 ? W1->w : nullptr;
   a.M = M;
@@ -771,7 +770,6 @@ int gemm(t5h_model* m, int kind, int epi, const Linear& W, const Linear* W1, con
     ReplayRec& r = m->replay[kind];
     r.type = ReplayRec::GEMM;
     r.epi = epi;
-    r.wfmt = W.fmt;
     r.ga = a;
     r.plan = plan;
   }
@@ -988,11 +986,11 @@ int run_block(t5h_model* m, int l, int T, int nwork, bool operand_ready = false,
     if (rc) return rc;
   }
   if (Ly.fused_qkv) {
-    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.qkv, nullptr, m->w.xn, D, T, m->w.qkvb, 0, 0, nw0, qkv_nl))) return rc;
+    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.qkv, nullptr, m->w.xn, T, m->w.qkvb, 0, 0, nw0, qkv_nl))) return rc;
   } else {
-    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.q, nullptr, m->w.xn, D, T, m->w.qkvb, 0, 0, nw0, qkv_nl))) return rc;
-    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.k, nullptr, m->w.xn, D, T, m->w.qkvb, 0, inner, nw0, qkv_nl))) return rc;
-    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.v, nullptr, m->w.xn, D, T, m->w.qkvb, 0, 2 * inner, nw0, qkv_nl)))
+    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.q, nullptr, m->w.xn, T, m->w.qkvb, 0, 0, nw0, qkv_nl))) return rc;
+    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.k, nullptr, m->w.xn, T, m->w.qkvb, 0, inner, nw0, qkv_nl))) return rc;
+    if ((rc = gemm(m, K_GEMM_QKV, EPI_QKV, Ly.v, nullptr, m->w.xn, T, m->w.qkvb, 0, 2 * inner, nw0, qkv_nl)))
       return rc;
   }
   {
@@ -1014,12 +1012,12 @@ int run_block(t5h_model* m, int l, int T, int nwork, bool operand_ready = false,
       r.D = c.d_kv;
     }
   }
-  if ((rc = gemm(m, K_GEMM_O, EPI_RESID, Ly.o, nullptr, m->w.ao, inner, T, m->w.x, D, 0, nullptr, fold ? &on : nullptr)))
+  if ((rc = gemm(m, K_GEMM_O, EPI_RESID, Ly.o, nullptr, m->w.ao, T, m->w.x, D, 0, nullptr, fold ? &on : nullptr)))
     return rc;
   const float* nw1 = nullptr;
   if (hybrid) {
     if ((rc = hybrid_linear(m, K_GEMM_GATE_UP, Ly.ln1, Ly.wi0, &Ly.wi1, T, nullptr, 0))) return rc;
-    return gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, c.d_ff, T, m->w.x, D, 0, nullptr,
+    return gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, T, m->w.x, D, 0, nullptr,
                 fold0 && next_gamma ? &wn : nullptr);
   }
   if (!fold) {
@@ -1069,23 +1067,23 @@ int run_block(t5h_model* m, int l, int T, int nwork, bool operand_ready = false,
       f2.rec_next += (size_t)t0 * 16;
       w2.rec += (size_t)t0 * 16;
       w2.nx += tiled_index(t0, 0, D);
-      if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn + tiled_index(t0, 0, D), D, n, m->w.hb,
+      if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn + tiled_index(t0, 0, D), n, m->w.hb,
                      c.d_ff, 0, nullptr, &f2)))
         return rc;
-      if ((rc = gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, c.d_ff, n, m->w.x + (size_t)t0 * D, D, 0,
+      if ((rc = gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, n, m->w.x + (size_t)t0 * D, D, 0,
                      nullptr, next_gamma ? &w2 : nullptr)))
         return rc;
     }
     return T5H_OK;
   }
   if (c.feed_forward_gated) {
-    if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn, D, T, m->w.hb, c.d_ff, 0, nw1, ffn_nl)))
+    if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn, T, m->w.hb, c.d_ff, 0, nw1, ffn_nl)))
       return rc;
   } else {
-    if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_RELU, Ly.wi0, nullptr, m->w.xn, D, T, m->w.hb, c.d_ff, 0, nw1, ffn_nl)))
+    if ((rc = gemm(m, K_GEMM_GATE_UP, EPI_RELU, Ly.wi0, nullptr, m->w.xn, T, m->w.hb, c.d_ff, 0, nw1, ffn_nl)))
       return rc;
   }
-  if ((rc = gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, c.d_ff, T, m->w.x, D, 0, nullptr,
+  if ((rc = gemm(m, K_GEMM_WO, EPI_RESID, Ly.wo, nullptr, m->w.hb, T, m->w.x, D, 0, nullptr,
                  fold && next_gamma ? &wn : nullptr)))
     return rc;
   return T5H_OK;
@@ -1253,7 +1251,7 @@ int enqueue_stack(t5h_model* m, const uint32_t* d_ids, int T, int nwork, float* 
       nwf = prenorm(m, m->final_ln, T, rc);
       if (rc) return rc;
     }
-    if ((rc = gemm(m, K_GEMM_PROJ, EPI_F32, m->proj, nullptr, m->w.xn, c.d_model, T, d_out, c.proj_dim, 0, nwf,
+    if ((rc = gemm(m, K_GEMM_PROJ, EPI_F32, m->proj, nullptr, m->w.xn, T, d_out, c.proj_dim, 0, nwf,
                    fold ? &pn : nullptr)))
       return rc;
   }
@@ -1914,9 +1912,9 @@ int t5h_ffn_block(t5h_model* m, int32_t layer, const float* x, int32_t T, float*
     rc = hybrid_linear(m, K_GEMM_GATE_UP, nullptr, Ly.wi0, &Ly.wi1, T, nullptr, 0);
   } else {
     HIP_OK(t5k::launch_f32_to_f16(m->w.x, m->w.xn, (size_t)T * c.d_model, c.d_model, m->stream));
-    rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn, c.d_model, T, m->w.hb, c.d_ff);
+    rc = gemm(m, K_GEMM_GATE_UP, EPI_GATED, Ly.wi0, &Ly.wi1, m->w.xn, T, m->w.hb, c.d_ff);
   }
-  if (!rc) rc = gemm(m, K_GEMM_WO, EPI_F32, Ly.wo, nullptr, m->w.hb, c.d_ff, T, m->w.x, c.d_model);
+  if (!rc) rc = gemm(m, K_GEMM_WO, EPI_F32, Ly.wo, nullptr, m->w.hb, T, m->w.x, c.d_model);
   m->batched_only = false;
   if (rc) return rc;
   HIP_OK(hipMemcpyAsync(y, m->w.x, bytes, hipMemcpyDeviceToHost, m->stream));
